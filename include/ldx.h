@@ -40,7 +40,7 @@ extern "C" {
 
 /* Message of the calling thread's most recent failure ("" if none). */
 const char* ldx_last_error(void);
-/* ABI version (12); bumped on any change to the structs below or the entry points. */
+/* ABI version (13); bumped on any change to the structs below or the entry points. */
 int ldx_abi_version(void);
 
 /* ---------------------------------------------------------------- conv3d -------
@@ -225,7 +225,8 @@ int ldx_group_norm_affine_moments_ws(const float* m0, int64_t chunks0, int32_t c
 /* GroupNorm statistics (as ldx_group_norm_affine) and LayerNorm (as ldx_layer_norm) of FP32
  * tensors, statistics in FP32 (per-thread Welford moments merged in a fixed order; the row
  * mean, then the mean squared deviation), FP32 output -- the FP32 networks' norms
- * (mlx_model.py:328-335, 360-367). No workspace. */
+ * (mlx_model.py:328-335, 360-367). No workspace: GroupNorm takes one workgroup per (group,
+ * batch item). */
 int ldx_group_norm_affine_f32(const float* x0, int64_t x0_pitch, int32_t c0, const float* x1, int64_t x1_pitch,
                               int32_t c1, int32_t batch, int64_t voxels, int32_t groups, const float* gamma,
                               const float* beta, float eps, float* affine, void* stream);

@@ -120,6 +120,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "ldx_packed_weight_exact_elems": (ctypes.c_size_t, [c_i32, c_i32, c_i32]),
     "ldx_group_norm_affine_f32": (c_i32, [c_vp, c_i64, c_i32, c_vp, c_i64, c_i32, c_i32, c_i64, c_i32,
                                           c_vp, c_vp, c_f32, c_vp, c_vp]),
+    "ldx_group_norm_f32_workspace_bytes": (ctypes.c_size_t, [c_i32, c_i64, c_i32, c_i32]),
+    "ldx_group_norm_affine_f32_ws": (c_i32, [c_vp, c_i64, c_i32, c_vp, c_i64, c_i32, c_i32, c_i64, c_i32,
+                                             c_vp, c_vp, c_f32, c_vp, c_vp, ctypes.c_size_t, c_vp]),
     "ldx_layer_norm_f32": (c_i32, [c_vp, c_i64, c_i64, c_i32, c_vp, c_vp, c_f32, c_vp, c_i64, c_vp]),
     "ldx_timestep_embedding_f32": (c_i32, [c_vp, c_i32, c_i32, c_vp, c_vp]),
     "ldx_vq_nearest4": (c_i32, [c_vp, c_vp, c_vp, c_vp, c_i64, c_i32, c_i32, c_vp, c_vp, c_vp]),
@@ -130,7 +133,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                            c_vp]),
 }
 
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 
 def _load() -> ctypes.CDLL:

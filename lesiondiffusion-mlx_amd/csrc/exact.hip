@@ -95,6 +95,99 @@ __global__ __launch_bounds__(256) void gn_f32_kernel(const float* __restrict__ x
   }
 }
 
+// Large FP32 tensors in two launches (gn_f32_kernel has one workgroup per (group, batch item):
+// 16 workgroups on 256 CUs for a 16-channel tensor, each of whose threads waits out a 4-byte
+// load and a division per value). Here a workgroup reduces `chunk` voxels over all channels,
+// so the reads are whole contiguous rows, and gn_finalize_kernel merges the chunks. A thread
+// owns V channels (16 bytes) of every vpi-th voxel, eight voxels' loads in flight: their mean,
+// then their squared deviations from it, merged into the running moments (Chan), one division
+// per eight voxels; no shift, no cancellation, and the order is fixed. Memory-bound; both
+// launches: 76 x 128 x 152 x 16 (95 MB) 2752 -> 22 us (4.3 TB/s), 128 x 160 x 160 x 96
+// (1.26 GB) 44.6 ms -> 215 us (5.9 TB/s), 19 x 32 x 38 x 64 89 -> 8.0 us.
+template <int V>
+__global__ __launch_bounds__(256) void gn_f32_partial_kernel(const float* __restrict__ x0, int64_t p0, int C0,
+                                                             const float* __restrict__ x1, int64_t p1, int C, int G,
+                                                             int64_t S, int64_t chunk, float* __restrict__ partial) {
+  typedef float vec __attribute__((ext_vector_type(V)));
+  __shared__ float s_n[256], s_mean[256 * V], s_m2[256 * V];   // per (voxel slot, channel)
+  const int b = blockIdx.y, t = threadIdx.x;
+  const int tpv = C / V, vpi = 256 / tpv, sub = t / tpv, c0 = (t % tpv) * V;
+  const bool active = sub < vpi;
+  const int64_t v_begin = (int64_t)blockIdx.x * chunk, v_end = min(S, v_begin + chunk);
+  const float* base = c0 < C0 ? x0 + c0 : x1 + (c0 - C0);
+  const int64_t pitch = c0 < C0 ? p0 : p1;
+  auto at = [&](int64_t v) { return *reinterpret_cast<const vec*>(base + ((int64_t)b * S + v) * pitch); };
+  float n = 0.f;
+  vec mean = (vec)(0.f), m2 = (vec)(0.f);
+  if (active) {
+    int64_t v = v_begin + sub;
+    for (; v + 7 * vpi < v_end; v += 8 * vpi) {
+      vec h[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) h[u] = at(v + u * vpi);
+      const vec bm = (((h[0] + h[1]) + (h[2] + h[3])) + ((h[4] + h[5]) + (h[6] + h[7]))) * 0.125f;
+      vec q = (vec)(0.f);
+#pragma unroll
+      for (int u = 0; u < 8; u++) q += (h[u] - bm) * (h[u] - bm);
+      const float f = 8.f / (n + 8.f);
+      const vec d = bm - mean;
+      mean += d * f;
+      m2 += q + d * d * (n * f);
+      n += 8.f;
+    }
+    for (; v < v_end; v += vpi) {
+      const vec d = at(v) - mean;
+      n += 1.f;
+      mean += d * (1.f / n);
+      m2 += d * d * ((n - 1.f) / n);
+    }
+  }
+  // The voxel slots' moments of a channel, folded in halves.
+  auto put = [&](int slot) {
+    if (t % tpv == 0) s_n[slot] = n;
+#pragma unroll
+    for (int e = 0; e < V; e++) { s_mean[slot * C + c0 + e] = mean[e]; s_m2[slot * C + c0 + e] = m2[e]; }
+  };
+  if (active) put(sub);
+  for (int k = vpi; k > 1;) {
+    const int half = (k + 1) / 2;
+    __syncthreads();
+    if (active && sub + half < k) {
+      const int o = sub + half;
+      const float on = s_n[o];
+      Moments m = {n, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < V; e++) {
+        m = merge(Moments{n, mean[e], m2[e]}, Moments{on, s_mean[o * C + c0 + e], s_m2[o * C + c0 + e]});
+        mean[e] = m.mean; m2[e] = m.m2;
+      }
+      n = m.n;
+      put(sub);
+    }
+    k = half;
+  }
+  __syncthreads();
+  const int gs = C / G;
+  for (int g = t; g < G; g += 256) {
+    Moments m = {0.f, 0.f, 0.f};
+    for (int c = g * gs; c < (g + 1) * gs; c++) m = merge(m, Moments{s_n[0], s_mean[c], s_m2[c]});
+    float* out = partial + (((int64_t)b * gridDim.x + blockIdx.x) * G + g) * 3;
+    out[0] = m.n; out[1] = m.mean; out[2] = m.m2;
+  }
+}
+
+// Voxels per workgroup of gn_f32_partial_kernel (0: the one-launch kernel). Whole
+// eight-voxel rounds of a workgroup, about four workgroups per CU. The one-launch kernel
+// stays for groups of fewer than 4,096 values, where a second launch costs what its 16
+// rounds per thread do: 3,200 values 6.9 us, 6,080 9.5 us, 8,192 11.8 us against 7.5 us.
+static int64_t gn_f32_chunk(int batch, int64_t voxels, int C, int groups) {
+  if (batch < 1 || voxels < 1 || C < 1 || groups < 1 || C % groups || C > 1024) return 0;
+  if (voxels * (C / groups) < 4096) return 0;
+  const int tpv = (C + 3) / 4;
+  const int64_t unit = 8 * (256 / tpv), want = ceil_div64(1024, batch);
+  return ceil_div64(ceil_div64(voxels, want), unit) * unit;
+}
+
 // One wave per row: mean, then the mean squared deviation, in FP32; the lanes' partial sums
 // added in a fixed butterfly order.
 __device__ __forceinline__ float wave_sum(float v) {
@@ -972,9 +1065,15 @@ int attention_f32(const ldx_attention_args* a, void* stream) {
 }
 }  // namespace ldx
 
-extern "C" int ldx_group_norm_affine_f32(const float* x0, int64_t x0_pitch, int32_t c0, const float* x1, int64_t x1_pitch,
-                                         int32_t c1, int32_t batch, int64_t voxels, int32_t groups, const float* gamma,
-                                         const float* beta, float eps, float* affine, void* stream) {
+extern "C" size_t ldx_group_norm_f32_workspace_bytes(int32_t batch, int64_t voxels, int32_t channels, int32_t groups) {
+  const int64_t chunk = gn_f32_chunk(batch, voxels, channels, groups);
+  return chunk ? (size_t)(batch * ceil_div64(voxels, chunk) * groups * 3) * sizeof(float) : 0;
+}
+
+extern "C" int ldx_group_norm_affine_f32_ws(const float* x0, int64_t x0_pitch, int32_t c0, const float* x1,
+                                            int64_t x1_pitch, int32_t c1, int32_t batch, int64_t voxels, int32_t groups,
+                                            const float* gamma, const float* beta, float eps, float* affine,
+                                            void* workspace, size_t workspace_bytes, void* stream) {
   if (!x0 || !gamma || !beta || !affine) return fail("group_norm_affine_f32: null pointer");
   if (c1 > 0 && !x1) return fail("group_norm_affine_f32: c1 > 0 but x1 is null");
   const int C = c0 + (c1 > 0 ? c1 : 0);
@@ -982,9 +1081,34 @@ extern "C" int ldx_group_norm_affine_f32(const float* x0, int64_t x0_pitch, int3
     return fail("group_norm_affine_f32: bad shape (batch %d voxels %lld C %d groups %d)", batch, (long long)voxels, C,
                 groups);
   if (x0_pitch < c0 || (c1 > 0 && x1_pitch < c1)) return fail("group_norm_affine_f32: pitch < channels");
-  hipLaunchKernelGGL(gn_f32_kernel, dim3(groups, batch), dim3(256), 0, as_stream(stream), x0, x0_pitch, c0,
-                     c1 > 0 ? x1 : x0, c1 > 0 ? x1_pitch : x0_pitch, C, groups, voxels, gamma, beta, eps, affine);
+  const float* xb = c1 > 0 ? x1 : x0;
+  const int64_t pb = c1 > 0 ? x1_pitch : x0_pitch;
+  hipStream_t st = as_stream(stream);
+  const bool vec = C % 4 == 0 && c0 % 4 == 0 && x0_pitch % 4 == 0 && pb % 4 == 0 && al16(x0) && al16(xb);
+  const size_t need = ldx_group_norm_f32_workspace_bytes(batch, voxels, C, groups);
+  if (need && workspace && workspace_bytes >= need && (vec || C <= 256)) {
+    const int64_t chunk = gn_f32_chunk(batch, voxels, C, groups), nchunks = ceil_div64(voxels, chunk);
+    const dim3 grid((unsigned)nchunks, batch);
+    float* part = (float*)workspace;
+    if (vec)
+      hipLaunchKernelGGL(gn_f32_partial_kernel<4>, grid, dim3(256), 0, st, x0, x0_pitch, c0, xb, pb, C, groups, voxels,
+                         chunk, part);
+    else
+      hipLaunchKernelGGL(gn_f32_partial_kernel<1>, grid, dim3(256), 0, st, x0, x0_pitch, c0, xb, pb, C, groups, voxels,
+                         chunk, part);
+    if (int rc = check_launch("group_norm_affine_f32: partial")) return rc;
+    return launch_gn_finalize(part, (int)nchunks, batch, C, groups, gamma, beta, eps, affine, st);
+  }
+  hipLaunchKernelGGL(gn_f32_kernel, dim3(groups, batch), dim3(256), 0, st, x0, x0_pitch, c0, xb, pb, C, groups, voxels,
+                     gamma, beta, eps, affine);
   return check_launch("group_norm_affine_f32");
+}
+
+extern "C" int ldx_group_norm_affine_f32(const float* x0, int64_t x0_pitch, int32_t c0, const float* x1, int64_t x1_pitch,
+                                         int32_t c1, int32_t batch, int64_t voxels, int32_t groups, const float* gamma,
+                                         const float* beta, float eps, float* affine, void* stream) {
+  return ldx_group_norm_affine_f32_ws(x0, x0_pitch, c0, x1, x1_pitch, c1, batch, voxels, groups, gamma, beta, eps,
+                                      affine, nullptr, 0, stream);
 }
 
 extern "C" int ldx_layer_norm_f32(const float* x, int64_t x_pitch, int64_t rows, int32_t features, const float* gamma,

@@ -235,6 +235,13 @@ __global__ __launch_bounds__(256) void gn_finalize_kernel(
   }
 }
 
+int launch_gn_finalize(const float* partial, int nchunks, int batch, int C, int groups, const float* gamma,
+                       const float* beta, float eps, float* affine, hipStream_t st) {
+  hipLaunchKernelGGL(gn_finalize_kernel, dim3(groups, batch), dim3(256), 0, st, partial, nchunks, C, groups, gamma,
+                     beta, eps, affine);
+  return check_launch("group_norm_affine: finalize");
+}
+
 // Small tensors (coarse UNet levels): one launch, one workgroup per (group, batch item).
 // Thread t sums (x - K) and (x - K)^2 over the group's channels of voxels t, t + 256, ...
 // with K the group's first value (a shift against cancellation), converts them to
@@ -534,7 +541,7 @@ __global__ void ddim_update_kernel(float* __restrict__ x, const f16* __restrict_
 using namespace ldx;
 
 extern "C" const char* ldx_last_error(void) { return g_error.c_str(); }
-extern "C" int ldx_abi_version(void) { return 12; }
+extern "C" int ldx_abi_version(void) { return 13; }
 
 extern "C" size_t ldx_packed_weight_elems(int32_t O, int32_t C, int32_t k, int32_t upsample) {
   if (O < 1 || C < 1 || (k != 1 && k != 3) || (upsample && k != 3)) return 0;
@@ -614,9 +621,7 @@ static int group_norm_affine_impl(const void* x0, int64_t p0, int32_t c0, const 
                        (int)nchunks);
   int rc = check_launch("group_norm_affine: partial");
   if (rc) return rc;
-  hipLaunchKernelGGL(gn_finalize_kernel, dim3(groups, batch), dim3(256), 0, st, part, (int)nchunks, C,
-                     groups, gamma, beta, eps, affine);
-  return check_launch("group_norm_affine: finalize");
+  return launch_gn_finalize(part, (int)nchunks, batch, C, groups, gamma, beta, eps, affine, st);
 }
 
 extern "C" int ldx_group_norm_affine(const void* x0, int64_t p0, int32_t c0, const void* x1,

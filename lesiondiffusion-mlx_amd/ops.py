@@ -440,8 +440,11 @@ def group_norm_affine(x: torch.Tensor, gamma: torch.Tensor, beta: torch.Tensor, 
     b32 = beta.to(torch.float32).contiguous()
     if x.dtype == torch.float32:
         out = torch.empty((b, c, 2), dtype=torch.float32, device=x.device)
-        check(lib.ldx_group_norm_affine_f32(_ptr(x), xp, c0, _ptr(x1), x1p, c1, b, d * h * w, groups, _ptr(g32),
-                                            _ptr(b32), float(eps), _ptr(out), _stream()), "group_norm_affine_f32")
+        ws_bytes = lib.ldx_group_norm_f32_workspace_bytes(b, d * h * w, c, groups)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
+        check(lib.ldx_group_norm_affine_f32_ws(_ptr(x), xp, c0, _ptr(x1), x1p, c1, b, d * h * w, groups, _ptr(g32),
+                                               _ptr(b32), float(eps), _ptr(out), _ptr(ws), ws_bytes, _stream()),
+              "group_norm_affine_f32")
         return out
     m0, m1 = moments_of(x), moments_of(x1)
     if m0 is not None and (x1 is None or m1 is not None) and (c // groups) % 2 == 0 and c0 % 2 == 0 \

@@ -197,6 +197,28 @@ def test_fp32_group_norm_and_layer_norm(pkg, dev) -> None:
                                rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize(("shape", "c1", "groups", "mean"), [
+    ((1, 8, 16, 32, 1), 0, 1, 0.0),      # the smallest group of the two-launch form, unaligned rows
+    ((1, 4, 9, 15, 32), 0, 32, 0.0),     # just below it
+    ((2, 17, 19, 23, 48), 16, 16, 50.0), # 12 threads per voxel (four idle), a group across both inputs
+    ((1, 16, 17, 19, 1024), 0, 32, 0.0), # one voxel slot per workgroup
+    ((1, 11, 13, 40, 6), 3, 3, -3.0),    # unaligned concat: one channel per thread
+    ((3, 21, 22, 23, 16), 0, 16, 1e3),   # one channel per group, mean >> deviation
+])
+def test_fp32_group_norm_of_large_tensors(pkg, dev, shape, c1, groups, mean) -> None:
+    """Bound: the offset beta - scale * mean carries scale * mean's rounding, so the absolute
+    part grows with |mean| / deviation (2^-20 of it: the mean's and the scale's few ulps)."""
+    rng = np.random.default_rng(6)
+    x = (rng.normal(size=shape) * 2 + mean).astype(np.float32)
+    c = shape[-1]
+    gamma, beta = rng.normal(size=c).astype(np.float32), rng.normal(size=c).astype(np.float32)
+    x0, x1 = dev32(x[..., :c - c1], dev), dev32(x[..., c - c1:], dev) if c1 else None
+    aff = host(pkg.ops.group_norm_affine(x0, dev32(gamma, dev), dev32(beta, dev), groups=groups, eps=1e-5, x1=x1))
+    want = onm.group_norm_affine(x.astype(np.float64).transpose(0, 4, 1, 2, 3), gamma.astype(np.float64),
+                                 beta.astype(np.float64), groups=groups, eps=1e-5)
+    np.testing.assert_allclose(aff, want, rtol=2e-6, atol=2e-6 + 2.0 ** -20 * abs(mean))
+
+
 @pytest.mark.parametrize(("lq", "lk", "d"), [(64, 3, 16), (300, 300, 32), (129, 77, 64), (8, 8, 16)])
 def test_fp32_attention_matches_float64(pkg, dev, lq, lk, d) -> None:
     rng = np.random.default_rng(lq + lk + d)
