@@ -60,6 +60,22 @@ __global__ void pack_weight_exact_kernel(const float* __restrict__ w, int O, int
   }
 }
 
+// v / (1 + exp(-v)) in fp32, within an ulp or two: exp(-v) = 2^n 2^f with n the nearest integer
+// to -v log2(e) and f the rest from log2(e) in two parts, and the quotient from the hardware
+// reciprocal with a Newton step, one residual correction and v_div_fixup (-0 for large
+// negative v, NaN for -inf, as the division gives). About 20 issue slots against about 45 of
+// expf and the compiler's division.
+__device__ __forceinline__ float silu32(float v) {
+  const float a = __builtin_amdgcn_fmed3f(v, -256.f, 256.f);
+  const float n = __builtin_rintf(a * -1.44269504f);
+  const float f = __builtin_fmaf(a, -1.92596299e-8f, __builtin_fmaf(a, -1.44269502f, -n));
+  const float d = 1.0f + __builtin_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
+  float r = __builtin_amdgcn_rcpf(d);
+  r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+  float q = v * r;
+  q = __builtin_fmaf(__builtin_fmaf(-q, d, v), r, q);
+  return __builtin_amdgcn_div_fixupf(q, d, v);
+}
 __device__ __forceinline__ float gelu_erf32(float v) { return v * (1.0f + erff(v * 0.70710678118654752f)) * 0.5f; }
 
 // ------------------------------------------------------------------ GroupNorm / LayerNorm
@@ -672,7 +688,7 @@ __global__ __launch_bounds__((ExactConvShape<KS, S, BD, BH, BW, KG, NCW>::NT)) v
     for (int e = 0; e < 4; e++) {
       float v = pre[k][e];
       if (p.affine) v = v * aff_s[e] + aff_o[e];
-      if (p.silu) v = v / (1.0f + expf(-v));
+      if (p.silu) v = silu32(v);
       if (!ok || c + e >= p.C) v = 0.f;
       asm volatile("" : "+v"(v));  // one value feeds both halves
       const f16 vh = (f16)v;
@@ -878,7 +894,7 @@ __global__ __launch_bounds__((ExactConvShape<KS, S, BD, BH, BW, KG, NCW>::NT)) v
         float u = (sum + add) * p.scale;
         if (p.res) u += p.res[ov * p.resp + o];
         if (p.act == LDX_ACT_GELU) u = gelu_erf32(u);
-        else if (p.act == LDX_ACT_SILU) u = u / (1.0f + expf(-u));
+        else if (p.act == LDX_ACT_SILU) u = silu32(u);
         t[r] = u;
       }
       float* yo = p.y + ov * p.yp + o0;
@@ -888,6 +904,230 @@ __global__ __launch_bounds__((ExactConvShape<KS, S, BD, BH, BW, KG, NCW>::NT)) v
 #pragma unroll
         for (int r = 0; r < 4; r++)
           if (o0 + r < p.O) yo[r] = t[r];
+      }
+    }
+  }
+}
+
+// ------------------------------------------------------------------ conv (narrow outputs)
+// The same conv with 32- or 16-row output tiles, where the 64-row tile above would spend half
+// or three quarters of its MFMAs on rows past O. A workgroup of four waves takes a brick of
+// BD x BH x BW output voxels (BW = 8: a 32-voxel MFMA column is four rows of eight) and 32
+// output channels (16: all of them), its halo staged 16 channels at a time.
+//
+// OT = 16 (O <= 16): the 32 rows of the A operand are the 16 rows of W_hi over the 16 of
+// W_lo, so one MFMA with x_hi gives hi x hi (rows 0-15) and lo x hi (rows 16-31) and a
+// second with x_lo gives hi x lo: two MFMAs instead of three for half the rows. The three
+// sums stay apart until the end, y = S_hh + (S_lh + S_hl) 2^-11. OT = 32: three MFMAs as
+// above. HS = 2 splits the hi x hi sum over taps 0-13 / 14-26, so that with more than one
+// chunk its chains are no longer than the two k-groups' above (same error against float64).
+//
+// LDS: per plane 16 bytes per (halo voxel, eight channels), unit 2 v + (half ^ (row & 1)):
+// the sixteen lanes that read together hold eight voxels of two neighbouring rows, and the
+// swapped halves put them in sixteen different bank groups. A tap's row parity flips the
+// halves. One buffer, and no register prefetch of the next chunk: three or four workgroups
+// share a CU and overlap one's staging with another's MFMAs (a prefetch cost the registers
+// of one of them: 162 -> 218 us). 76 x 128 x 152, 16 -> 16, GroupNorm + SiLU: 854 -> 151 us,
+// 1.3 TB/s; bound by the VALU of the prologue (every value prepared 600 / 256 = 2.3 times,
+// about 45 us), LDS reads (2 KB per column and tap, about 36 us) and MFMAs (36 us), which
+// overlap only in part.
+template <int OT, int BD, int BH, int HS>
+struct NarrowConvShape {
+  static constexpr int BW = 8, HD = BD + 2, HH = BH + 2, HW = BW + 2, NHV = HD * HH * HW;
+  static constexpr int NCW = BD * BH * BW / 128;               // 32-voxel columns per wave
+  static constexpr int NIT = (NHV * 2 + 255) / 256;            // staging items (8 channels) per thread
+  static constexpr int PL = NHV * 16;                          // halves per plane
+  static_assert((OT == 16 || OT == 32) && (HS == 1 || HS == 2), "16 or 32 output rows, one or two hi x hi sums");
+  static_assert(BH % 4 == 0 && BD * BH * BW % 128 == 0, "whole columns per wave");
+};
+
+template <int OT, int BD, int BH, int HS>
+__global__ __launch_bounds__(256, BH == 4 && OT * HS < 64 ? 4 : 3) void conv3d_exact_narrow_kernel(ExactConvParams p) {
+  touch_args(p);
+  using SH = NarrowConvShape<OT, BD, BH, HS>;
+  constexpr int NCW = SH::NCW, NIT = SH::NIT, PL = SH::PL, BW = SH::BW, HW = SH::HW, HH = SH::HH;
+  extern __shared__ __align__(16) f16 smem[];   // [hi, lo][PL]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, g = tid & 1;
+  int r;   // contiguous brick ranges per XCD, whose halos then meet in its L2
+  {
+    const int n = gridDim.x, l = blockIdx.x, per = n >> 3, rem = n & 7, x = l & 7, k = l >> 3;
+    r = x < rem ? x * (per + 1) + k : rem * (per + 1) + (x - rem) * per + k;
+  }
+  const int bw = r % p.nbw; r /= p.nbw;
+  const int bh = r % p.nbh; r /= p.nbh;
+  const int b = r / p.nbd, od0 = (r % p.nbd) * BD, oh0 = bh * BH, ow0 = bw * BW;
+
+  // Item i = tid + 256 k: halo voxel i / 2, channels 8 (i % 2) .. + 7 of the chunk. Voxels in
+  // the padding and channels past C get an offset past the buffer resource and read zeros,
+  // so the loads need no branch. The resource starts at the halo's first source plane; a
+  // 16-channel chunk lies in one of the two inputs (C0 % 16 == 0 with a second input).
+  f32x4 pre[NIT][2];
+  f32x4 aff[4];   // (scale, offset) pairs of the thread's eight channels
+  int vox[NIT];   // source voxel from that plane, or -1
+  const int sd0 = max(od0 - 1, 0) >> p.up;
+#pragma unroll
+  for (int k = 0; k < NIT; k++) {
+    const int hv = (tid + 256 * k) >> 1;
+    const int rd = od0 - 1 + hv / (HH * HW), rh = oh0 - 1 + (hv / HW) % HH, rw = ow0 - 1 + hv % HW;
+    const bool in = hv < SH::NHV && (unsigned)rd < (unsigned)p.RD && (unsigned)rh < (unsigned)p.RH &&
+                    (unsigned)rw < (unsigned)p.RW;
+    vox[k] = in ? (((rd >> p.up) - sd0) * p.IH + (rh >> p.up)) * p.IW + (rw >> p.up) : -1;
+  }
+  auto load_chunk = [&](int kc) {
+    const int c = kc * 16 + g * 8;
+    const bool in0 = kc * 16 < p.C0;
+    const int pitch = (int)(in0 ? p.p0 : p.p1), cl = in0 ? c : c - p.C0, cn = in0 ? p.C0 : p.C - p.C0;
+    const float* base = (in0 ? p.x0 : p.x1) + ((int64_t)b * p.ID + sd0) * p.IH * p.IW * pitch;
+    const int64_t left = ((int64_t)(p.ID - sd0) * p.IH * p.IW * pitch - pitch + cn) * 4;
+    const auto rs = make_rsrc(base, left < 0xffffff00ll ? (unsigned)left : 0xffffff00u);
+    if (p.affine) {
+      const auto ra = make_rsrc(p.affine + (int64_t)b * p.C * 2, (unsigned)p.C * 8);
+#pragma unroll
+      for (int i = 0; i < 4; i++) aff[i] = buffer_load16<f32x4>(ra, (unsigned)c * 8 + 16 * i);
+    }
+#pragma unroll
+    for (int k = 0; k < NIT; k++)
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+        pre[k][q] = buffer_load16<f32x4>(
+            rs, vox[k] >= 0 && cl + 4 * q < cn ? ((unsigned)vox[k] * (unsigned)pitch + (unsigned)(cl + 4 * q)) * 4u : 0xffffff00u);
+  };
+  auto store_chunk = [&](int kc) {
+    const int c = kc * 16 + g * 8;
+#pragma unroll
+    for (int k = 0; k < NIT; k++) {
+      const int hv = (tid + 256 * k) >> 1;
+      if (hv >= SH::NHV) continue;
+      f16x8 h8, l8;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        float v = pre[k][e >> 2][e & 3];
+        if (p.affine) v = v * aff[e >> 1][2 * (e & 1)] + aff[e >> 1][2 * (e & 1) + 1];
+        if (p.silu) v = silu32(v);
+        if (vox[k] < 0 || c + e >= p.C) v = 0.f;
+        asm volatile("" : "+v"(v));  // one value feeds both halves
+        const f16 vh = (f16)v;
+        h8[e] = vh;
+        l8[e] = (f16)((v - (float)vh) * 2048.0f);
+      }
+      f16* dst = smem + (2 * hv + (g ^ ((hv / HW) & 1))) * 8;   // HH is even: (hv / HW) & 1 is the row's parity
+      *reinterpret_cast<f16x8*>(dst) = h8;
+      *reinterpret_cast<f16x8*>(dst + PL) = l8;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  static_assert(HH % 2 == 0, "row parity");
+
+  // Column j of this wave starts at brick voxel (wave + 4 j) * 32.
+  int hb[NCW], par[NCW];
+#pragma unroll
+  for (int j = 0; j < NCW; j++) {
+    const int v = (wave + 4 * j) * 32 + (lane & 31);
+    const int ld = v / (BH * BW), lh = (v / BW) % BH, lw = v % BW;
+    const int hv = (ld * HH + lh) * HW + lw;
+    hb[j] = 2 * hv * 8;
+    par[j] = (half ^ (lh & 1)) * 8;
+  }
+
+  // A fragment of a tap: rows as packed (OT = 32), or W_hi rows 0-15 over W_lo rows 0-15.
+  const f16* wrow;
+  if constexpr (OT == 16)
+    wrow = p.w + ((lane & 16) ? p.wplane : 0) + ((lane & 15) + 32 * half) * 8;
+  else
+    wrow = p.w + (int64_t)blockIdx.y * p.NKC * 27 * 512 + lane * 8;
+  f16x8 ah[3], al[3];
+  auto load_w = [&](int kc, int t, int slot) {
+    const f16* q = wrow + ((int64_t)kc * 27 + t) * 512;
+    ah[slot] = *reinterpret_cast<const f16x8*>(q);
+    if constexpr (OT == 32) al[slot] = *reinterpret_cast<const f16x8*>(q + p.wplane);
+  };
+
+  f32x16 acc_h[HS][NCW], acc_x[NCW];
+#pragma unroll
+  for (int j = 0; j < NCW; j++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc_h[0][j][e] = acc_h[HS - 1][j][e] = acc_x[j][e] = 0.f;
+
+  load_w(0, 0, 0);
+  load_w(0, 1, 1);
+  for (int kc = 0; kc < p.NCH; kc++) {
+    load_chunk(kc);
+    if (kc) __syncthreads();   // the previous chunk is read
+    store_chunk(kc);
+    __syncthreads();
+    const bool more = kc + 1 < p.NCH;
+#pragma unroll
+    for (int t = 0; t < 27; t++) {
+      if (t + 2 < 27) load_w(kc, t + 2, (t + 2) % 3);
+      else if (more) load_w(kc + 1, t + 2 - 27, (t + 2) % 3);
+      const int kh = (t / 3) % 3, toff = ((t / 9) * HH + kh) * HW + t % 3;
+      f16x8 xh[NCW], xl[NCW];
+#pragma unroll
+      for (int j = 0; j < NCW; j++) {
+        const f16* q = smem + hb[j] + ((kh & 1) ? 8 - par[j] : par[j]) + toff * 16;
+        xh[j] = *reinterpret_cast<const f16x8*>(q);
+        xl[j] = *reinterpret_cast<const f16x8*>(q + PL);
+      }
+      const int s = t % 3, u = t < 14 ? 0 : HS - 1;
+#pragma unroll
+      for (int j = 0; j < NCW; j++) acc_h[u][j] = mfma_h(ah[s], xh[j], acc_h[u][j]);
+#pragma unroll
+      for (int j = 0; j < NCW; j++) acc_x[j] = mfma_h(ah[s], xl[j], acc_x[j]);
+      if constexpr (OT == 32) {
+#pragma unroll
+        for (int j = 0; j < NCW; j++) acc_x[j] = mfma_h(al[s], xh[j], acc_x[j]);
+      }
+    }
+  }
+
+  // Lane (half, col): voxel col of its columns, channels 8 q + 4 half + r in element 4 q + r
+  // (OT = 16: q < 2, the lo x hi sums of the same channels eight elements on).
+  const int ob0 = OT == 32 ? blockIdx.y * 32 : 0;
+  f32x4 add[OT / 8];
+#pragma unroll
+  for (int q = 0; q < OT / 8; q++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int o = min(ob0 + 8 * q + 4 * half + e, p.O - 1);
+      add[q][e] = p.bias ? p.bias[(p.bias_batched ? (int64_t)b * p.O : 0) + o] : 0.f;
+      if (p.shift) add[q][e] += p.shift[(int64_t)b * p.shiftp + o];
+    }
+#pragma unroll
+  for (int j = 0; j < NCW; j++) {
+    const int v = (wave + 4 * j) * 32 + (lane & 31);
+    const int od = od0 + v / (BH * BW), oh = oh0 + (v / BW) % BH, ow = ow0 + v % BW;
+    if (od >= p.OD || oh >= p.OH || ow >= p.OW) continue;
+    const int64_t ov = (((int64_t)b * p.OD + od) * p.OH + oh) * p.OW + ow;
+    f32x16 sh = acc_h[0][j];
+    if constexpr (HS == 2) sh += acc_h[1][j];
+#pragma unroll
+    for (int q = 0; q < OT / 8; q++) {
+      const int o0 = ob0 + 8 * q + 4 * half;
+      if (o0 >= p.O) continue;
+      f32x4 t;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float cross = OT == 16 ? sh[(4 * q + e + 8) & 15] + acc_x[j][4 * q + e] : acc_x[j][4 * q + e];
+        t[e] = (sh[4 * q + e] + cross * (1.0f / 2048.0f) + add[q][e]) * p.scale;
+      }
+      if (p.vec_out && o0 + 3 < p.O) {
+        if (p.res) t += *reinterpret_cast<const f32x4*>(p.res + ov * p.resp + o0);
+      } else if (p.res) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) t[e] += p.res[ov * p.resp + min(o0 + e, p.O - 1)];
+      }
+      if (p.act) {
+#pragma unroll 1
+        for (int e = 0; e < 4; e++) t[e] = p.act == LDX_ACT_GELU ? gelu_erf32(t[e]) : silu32(t[e]);
+      }
+      float* yo = p.y + ov * p.yp + o0;
+      if (p.vec_out && o0 + 3 < p.O) {
+        *reinterpret_cast<f32x4*>(yo) = t;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (o0 + e < p.O) yo[e] = t[e];
       }
     }
   }
@@ -953,6 +1193,19 @@ static int launch_exact(ExactConvParams p, int64_t bricks, hipStream_t st) {
   return check_launch("conv3d (fp32)");
 }
 
+template <int OT, int BD, int BH, int HS>
+static int launch_narrow(ExactConvParams p, int64_t bricks, hipStream_t st) {
+  using SH = NarrowConvShape<OT, BD, BH, HS>;
+  auto kern = conv3d_exact_narrow_kernel<OT, BD, BH, HS>;
+  const int lds = SH::PL * 4;
+  p.NCH = (p.C + 15) / 16;
+  if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return fail("conv3d (fp32): cannot reserve %d bytes of LDS", lds);
+  if (bricks >= (1ll << 31)) return fail("conv3d (fp32): grid too large");
+  hipLaunchKernelGGL(kern, dim3((unsigned)bricks, (unsigned)((p.O + OT - 1) / OT)), dim3(256), lds, st, p);
+  return check_launch("conv3d (fp32)");
+}
+
 static bool al16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
 int conv3d_exact(const ldx_conv3d_args* a, void* stream) {
@@ -1004,6 +1257,25 @@ int conv3d_exact(const ldx_conv3d_args* a, void* stream) {
   if (a->stride == 2) {
     nb = bricks(2, 4, 4);
     return launch_exact<3, 2, 2, 4, 4, 2, 1>(p, nb, st);
+  }
+  // An odd number of 32-channel output blocks leaves the 64-row tile half empty (O <= 16:
+  // three quarters): those take the 32- / 16-row kernel from 64 bricks on (its loads need
+  // 16-byte rows, a concat on a 16-channel boundary and 31-bit offsets over a halo's planes).
+  // us, 64-row tile / narrow, GroupNorm + SiLU and residual: 76x128x152 16->16 854 / 151 and
+  // 32->16 873 / 273; 38x64x76 32->32 147 / 64; 19x32x38 64->32 32 / 26; 20x24x24 32->32
+  // 25 / 16; 40x64x64 96->96 438 / 345. Whole pairs of blocks stay: 19x32x38 128->64 60 / 72,
+  // 40x64x64 128->128 567 / 587.
+  const int64_t span = 10ll * a->in_h * a->in_w * (a->x0_pitch > p.p1 ? a->x0_pitch : p.p1) * 4;
+  if ((O + 31) / 32 % 2 == 1 && p.vec_in && (!p.vec_out || !p.res || (a->residual_pitch % 4 == 0 && al16(p.res))) &&
+      (a->c1 == 0 || a->c0 % 16 == 0) && span < (1ll << 31)) {
+    if (C <= 16 && O <= 16) {
+      nb = bricks(4, 8, 8);
+      if (nb >= 64) return launch_narrow<16, 4, 8, 1>(p, nb, st);
+    }
+    nb = bricks(4, 4, 8);
+    if (nb >= 64)
+      return O <= 16 ? launch_narrow<16, 4, 4, 2>(p, nb, st)
+             : C <= 16 ? launch_narrow<32, 4, 4, 1>(p, nb, st) : launch_narrow<32, 4, 4, 2>(p, nb, st);
   }
   nb = bricks(4, 4, 8);
   if (nb * oblocks >= 128) return launch_exact<3, 1, 4, 4, 8, 2, 2>(p, nb, st);

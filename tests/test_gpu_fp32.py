@@ -139,6 +139,54 @@ def test_fp32_exact_conv_tilings_with_group_norm_prologue(pkg, dev, shape, out_c
     assert_near_fp32(host(y).transpose(0, 4, 1, 2, 3), expected, mag, extra=4 * 2.0 ** -23)
 
 
+@pytest.mark.parametrize(("shape", "c0", "out_c", "up", "act"), [
+    ((1, 16, 17, 33, 65), 16, 16, False, None),    # 16 rows, one chunk; partial bricks on every axis
+    ((2, 16, 9, 23, 41), 16, 3, False, "silu"),    # a partial output quad
+    ((1, 48, 13, 19, 61), 16, 16, False, None),    # concat: three chunks from two inputs
+    ((1, 36, 13, 19, 61), 32, 32, False, "gelu"),  # a chunk of four channels
+    ((1, 8, 16, 17, 57), 8, 32, False, None),      # half a chunk, 32 rows
+    ((1, 20, 5, 9, 17), 20, 32, True, None),       # the upsampled grid
+    ((1, 64, 16, 16, 36), 32, 96, False, None),    # three row blocks
+])
+def test_fp32_narrow_output_conv(pkg, dev, shape, c0, out_c, up, act) -> None:
+    """The 16- and 32-row tiles (at least 64 bricks of 4 x 4 x 8) at the exact-mode bound,
+    through the GroupNorm affine + SiLU prologue and the whole epilogue."""
+    x, w, _ = fp32_case(shape, out_c, sum(shape) + out_c)
+    rng = np.random.default_rng(out_c + c0)
+    n, c = shape[:2]
+    aff = np.stack([rng.normal(size=(n, c)), rng.normal(size=(n, c)) * 0.3], -1).astype(np.float32).astype(np.float64)
+    grid = tuple(2 * v for v in shape[2:]) if up else shape[2:]
+    bias, shift = (rng.normal(size=(n, out_c)).astype(np.float32).astype(np.float64) for _ in range(2))
+    res = rng.normal(size=(n, out_c) + grid).astype(np.float32).astype(np.float64)
+    xd = ndhwc(x)
+    pack = pkg.ops.pack_upsample_weight if up else pkg.ops.pack_weight
+    y = pkg.ops.nax_conv3d(dev32(xd[..., :c0], dev), pack(dev32(w, dev)), dev32(bias, dev), upsample=up,
+                           x1=dev32(xd[..., c0:], dev) if c0 < c else None, affine=dev32(aff, dev), silu=True,
+                           shift=dev32(shift, dev), residual=dev32(ndhwc(res), dev), output_scale=0.5, act=act)
+    torch.cuda.synchronize()
+    prep = onm.silu(onm.apply_affine(x, aff))
+    prep = ocv.upsample_nearest2(prep) if up else prep
+    expected = ocv.conv3d(prep, w, bias + shift) * 0.5 + res
+    mag = ocv.conv3d_magnitude(prep, w, bias + shift) * 0.5 + np.abs(res)
+    if act:   # both have slopes below 1.13; their fp32 evaluation adds a few ulps
+        expected = onm.gelu(expected) if act == "gelu" else onm.silu(expected)
+        mag = 1.13 * mag + 4 * np.abs(expected)
+    assert_near_fp32(host(y).transpose(0, 4, 1, 2, 3), expected, mag, extra=4 * 2.0 ** -23)
+
+
+def test_fp32_silu_of_extreme_values(pkg, dev) -> None:
+    """silu(v) through the prologue of a 1x1x1 identity conv: from where exp(-v) underflows to
+    where it overflows, as v / (1 + exp(-v)) gives it (large negative v: 0), within 4 ulps."""
+    v = np.array([0.0, 1e-30, -1e-30, 0.5, -0.5, 17.25, -17.25, 87.0, -87.0, 89.5, -89.5, -104.0, 300.0, -300.0, 6e4,
+                  -6e4], np.float32)
+    x = torch.from_numpy(np.tile(v, (1, 1, 1, 4, 1))).to(dev)
+    y = pkg.ops.nax_conv3d(x, pkg.ops.pack_weight(torch.eye(16, device=dev)), silu=True)
+    with np.errstate(over="ignore"):
+        want = v.astype(np.float64) / (1 + np.exp(-v.astype(np.float64)))
+    # the split keeps 22 bits and is absolute below 2^-24 (fp16's subnormal step over 2^11)
+    np.testing.assert_allclose(host(y)[0, 0, 0, 0], want, rtol=4 * 2.0 ** -22, atol=2.0 ** -35)
+
+
 @pytest.mark.parametrize("k", [1, 3])
 def test_fp32_unaligned_concat_with_batched_affine(pkg, dev, k) -> None:
     """Channel counts that are not multiples of 4 (element-wise input reads), two batch items
