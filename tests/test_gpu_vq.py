@@ -104,6 +104,26 @@ def test_config_sized_search_on_sampled_rows(pkg, dev, dtype) -> None:
     np.testing.assert_array_equal(_bits(q[rows]), _bits(want_q))
 
 
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize(("positions", "entries"), [(81920, 64), (82001, 2049), (81919, 4130), (97, 6143), (33, 65)])
+def test_search_edges_of_chunks_and_schedules(pkg, dev, dtype, positions, entries) -> None:
+    """Both schedules around their boundary (81,920 positions) and code counts around the
+    64-code chunks and 2,048-code stages; duplicates across chunks, values near zero and large,
+    an all-zero and a non-finite latent: sampled rows and the last ones equal the oracle."""
+    tt, nt = DTYPES[dtype]
+    rng = np.random.default_rng(positions + entries)
+    cb = (rng.normal(size=(entries, 4)) * np.exp2(rng.integers(-12, 5, (entries, 1)))).astype(nt)
+    cb[-1] = cb[entries // 2] = cb[1]
+    flat = (rng.normal(size=(positions, 4)) * np.exp2(rng.integers(-12, 5, (positions, 1)))).astype(nt)
+    flat[-1], flat[-2], flat[-3], flat[-4] = cb[1], 0, cb[-2], np.inf
+    idx, q, _ = _search(pkg, dev, flat, cb, tt)
+    rows = np.unique(np.concatenate([[0], positions - 1 - np.arange(32), rng.integers(0, positions, 512)]))
+    with np.errstate(invalid="ignore", over="ignore"):
+        want_idx, want_q = ovq.quantize4(flat[rows], cb, nt)
+    np.testing.assert_array_equal(idx[rows], want_idx)
+    np.testing.assert_array_equal(_bits(q[rows][:-4]), _bits(want_q[:-4]))
+
+
 def test_search_rejects_bad_arguments(pkg, dev) -> None:
     """Shape and dtype errors raise before anything is launched."""
     z = torch.zeros((3, 4), dtype=torch.float16, device=dev)
