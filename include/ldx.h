@@ -252,10 +252,12 @@ int ldx_layer_norm(const void* x, int64_t x_pitch, int64_t rows, int32_t feature
  * broadcast axis; -inf removes a key; a query row with every key removed gives 0.
  * LDX_DTYPE_F32 (the FP32 networks; the reference's FP32 attention, _attention.py:52-145):
  * head_dim 16, 32 or 64, no mask, FP32 scores, probabilities and products throughout.
- * V is read as it lies and transposed by the LDS reads. Scratch memory serves one plan
- * only: wide heads (128, 256) whose 128-query tiles spread unevenly over the CUs (the VQ
- * decoder's 51,200-token mid attention: 400 tiles on 256 CUs) split each tile's keys into
- * equal pieces, one workgroup each, and merge the pieces' partial states in a second
+ * V is read as it lies and transposed by the LDS reads. Scratch memory serves two plans:
+ * FP32 with heads of 32 or 64 and at least 609 keys writes K and V once as hi / lo fp16
+ * operands there and splits the keys into ranges; and wide heads (128, 256) whose 128-query
+ * tiles spread unevenly over the CUs (the VQ decoder's 51,200-token mid attention: 400 tiles
+ * on 256 CUs) split each tile's keys into equal pieces, one workgroup each. Either merges the
+ * pieces' partial states in a last
  * launch; ldx_attention_workspace_bytes returns their size (0 for every other plan). A
  * NULL or smaller workspace runs one workgroup per tile instead (same results within
  * fp32 summation order). */

@@ -1439,13 +1439,15 @@ namespace bf16_path {
 size_t attention_workspace_bytes(const ldx_attention_args* a);
 int attention_entry(const ldx_attention_args* a, void* stream);
 }  // namespace bf16_path
-int attention_f32(const ldx_attention_args* a, void* stream);   // exact.hip
+size_t attention_f32_workspace_bytes(const ldx_attention_args* a);   // exact.hip
+int attention_f32(const ldx_attention_args* a, void* stream);
 }  // namespace ldx
 
 // The C entry points (in the fp16 unit only): the kernels of the args' dtype.
 extern "C" size_t ldx_attention_workspace_bytes(const ldx_attention_args* a) {
   if (a && a->dtype == LDX_DTYPE_BF16) return ldx::bf16_path::attention_workspace_bytes(a);
   if (a && a->dtype == LDX_DTYPE_F16) return ldx::f16_path::attention_workspace_bytes(a);
+  if (a && a->dtype == LDX_DTYPE_F32) return ldx::attention_f32_workspace_bytes(a);
   return 0;
 }
 

@@ -532,6 +532,263 @@ __global__ __launch_bounds__(256) void attention_split_kernel(SplitAttnParams p)
   }
 }
 
+// Long FP32 sequences, the same split form in three launches. The kernel above splits K and V
+// again for every 128 queries (32 VALU operations per wave and block) and has one workgroup per
+// 128 queries (LMNet's 23,104 tokens x 2 heads: 362 on 256 CUs, so some run two). Here
+// split_kv_kernel writes K and V once as hi / lo MFMA operands in fragment order,
+// attention_planes_kernel takes them by DMA (no VALU, no transposition) over one of S equal key
+// ranges per workgroup, and attention_planes_merge_kernel merges the ranges' states.
+//
+// Softmax: the base moves only when a lane's 16 probabilities sum to 128 (a score about 7 above
+// it), seen on the sum that is needed anyway, so that no maximum is taken and the accumulators
+// are rarely rescaled; the block's probabilities are then made again. Probabilities are kept as p 2^8 (scaled after exp2: in its argument the 8 would cost
+// three of its bits, 2.0e-7 -> 2.9e-7 against float64): hi = half(p), lo = half(p - hi) unscaled,
+// one v_cvt and one mixed fused multiply-add; what lo loses to fp16's subnormal step is below
+// 2^-32 of the largest probability. Ph Vh, Pl Vh and 2^11 Ph Vl have an accumulator each.
+// Per 32 x 32 block 12 (D = 32) MFMAs and about 110 VALU operations, 16 of them exp2; VALU-bound.
+// 23,104 tokens, two 32-wide heads: 1250 -> 479 us (285 TFLOP/s of FP32 products).
+struct PlanesAttnParams {
+  int B, H, L, LK, nblk, S, per;   // key blocks of 32, key ranges, blocks per range
+  const float* q; int64_t qs0, qs1, qs2;
+  const float* k; int64_t ks0, ks1, ks2;
+  const float* v; int64_t vs0, vs1, vs2;
+  float* o; int64_t os0, os1, os2;
+  float c;          // scale * log2(e)
+  f16* planes;      // [batch * head][block][Kh, Kl: D / 16 each; Vh, Vl: 2 D / 32 each][64][8]
+  float* part;      // [query tile, batch * head][range][wave][D / 4 + 1][32] float4 (O, then (mb, l)); S > 1
+};
+
+// Fragments of a 32-key block: K rows permuted by split_key_row (lane l: key row l % 32, dims
+// 16 dk + 8 (l / 32) + e), V^T rows = dims (lane l: dim 32 db + l % 32, keys 16 ks + 8 (l / 32) + e).
+template <int D>
+__global__ __launch_bounds__(256) void split_kv_kernel(PlanesAttnParams p) {
+  touch_args(p);
+  constexpr int NF = D / 16;   // fragments of K (per plane); as many of V: 2 k-steps x D / 32
+  const int blk = blockIdx.x, bh = blockIdx.y, b = bh / p.H, h = bh % p.H;
+  const float* kp = p.k + (int64_t)b * p.ks0 + (int64_t)h * p.ks2;
+  const float* vp = p.v + (int64_t)b * p.vs0 + (int64_t)h * p.vs2;
+  f16* out = p.planes + ((int64_t)bh * p.nblk + blk) * (4 * NF * 512);
+  for (int i = threadIdx.x; i < 2 * NF * 64; i += 256) {
+    const int l = i & 63, f = (i >> 6) % NF, isv = i / (NF * 64), r = l & 31, hf = l >> 5;
+    float x[8];
+    if (!isv) {
+      const int key = blk * 32 + split_key_row(r);
+#pragma unroll
+      for (int e = 0; e < 8; e++) x[e] = key < p.LK ? kp[(int64_t)key * p.ks1 + f * 16 + 8 * hf + e] : 0.f;
+    } else {
+      const int ks = f / (D / 32), db = f % (D / 32);
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const int key = blk * 32 + 16 * ks + 8 * hf + e;
+        x[e] = key < p.LK ? vp[(int64_t)key * p.vs1 + db * 32 + r] : 0.f;
+      }
+    }
+    f16x8 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      hi[e] = (f16)x[e];
+      lo[e] = (f16)((x[e] - (float)hi[e]) * 2048.0f);
+    }
+    f16* dst = out + ((isv ? 2 * NF : 0) + f) * 512 + l * 8;
+    *reinterpret_cast<f16x8*>(dst) = hi;
+    *reinterpret_cast<f16x8*>(dst + NF * 512) = lo;
+  }
+}
+
+template <int D>
+__global__ __launch_bounds__(256, D == 32 ? 4 : 2) void attention_planes_kernel(PlanesAttnParams p) {
+  touch_args(p);
+  constexpr int NF = D / 16, DB = D / 32, BLK = 4 * NF * 512;   // halves per block
+  constexpr int RING = 3;
+  __shared__ __attribute__((aligned(16))) f16 smem[RING * BLK];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hf = lane >> 5, col = lane & 31;
+  int wg;   // contiguous runs per XCD: the query tiles of one (batch, head, range) read the same keys
+  {
+    const int n = gridDim.x, l = blockIdx.x, per = n >> 3, rem = n & 7, x = l & 7, k = l >> 3;
+    wg = x < rem ? x * (per + 1) + k : rem * (per + 1) + (x - rem) * per + k;
+  }
+  const int nq = (p.L + 127) / 128;
+  const int qt = wg % nq, range = (wg / nq) % p.S, bh = wg / nq / p.S, b = bh / p.H, h = bh % p.H;
+  const int blk0 = range * p.per, nb = min(p.per, p.nblk - blk0);
+  const f16* src = p.planes + ((int64_t)bh * p.nblk + blk0) * BLK;
+
+  const int q0 = qt * 128 + wave * 32, qi = min(q0 + col, p.L - 1);
+  const float* qb = p.q + (int64_t)b * p.qs0 + (int64_t)h * p.qs2 + (int64_t)qi * p.qs1;
+  f16x8 qh[NF], ql[NF];
+#pragma unroll
+  for (int dk = 0; dk < NF; dk++) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(qb + dk * 16 + 8 * hf);
+    const f32x4 c4 = *reinterpret_cast<const f32x4*>(qb + dk * 16 + 8 * hf + 4);
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      float x = (e < 4 ? a[e] : c4[e - 4]) * p.c;
+      asm volatile("" : "+v"(x));   // one fp32 value feeds both halves
+      qh[dk][e] = (f16)x;
+      ql[dk][e] = (f16)((x - (float)qh[dk][e]) * 2048.0f);
+    }
+  }
+  vmcnt_wait<0>();   // from here on only the DMAs below are counted
+
+  // Wave w copies its quarter of a block: NF kilobytes, NF DMAs.
+  auto dma = [&](int it) {
+    const f16* s = src + (int64_t)it * BLK + wave * (NF * 512) + lane * 8;
+    const unsigned d = lds_offset(smem + (it % RING) * BLK + wave * (NF * 512));
+#pragma unroll
+    for (int i = 0; i < NF; i++) dma_b128(s + i * 512, d + i * 1024);
+  };
+  auto frag = [&](int slot, int f) { return *reinterpret_cast<const f16x8*>(smem + slot * BLK + f * 512 + lane * 8); };
+
+  f32x16 oh[DB], ol[DB], ox[DB];
+#pragma unroll
+  for (int i = 0; i < DB; i++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) oh[i][e] = ol[i][e] = ox[i][e] = 0.f;
+  float mb = -1e30f, l = 0.f;
+  dma(0);
+  if (nb > 1) dma(1);
+  for (int it = 0; it < nb; it++) {
+    // This wave's share of block it has landed when at most block it + 1's DMAs are outstanding;
+    // after the barrier so have the others', and the slot of block it - 1 is free.
+    if (it + 1 < nb) vmcnt_wait<NF>();
+    else vmcnt_wait<0>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (it + 2 < nb) dma(it + 2);
+    const int slot = it % RING;
+    f32x16 sh = {}, sx = {};
+#pragma unroll
+    for (int dk = 0; dk < NF; dk++) {
+      const f16x8 kh = frag(slot, dk), kl = frag(slot, NF + dk);
+      sh = mfma_h(kh, qh[dk], sh);
+      sx = mfma_h(kh, ql[dk], sx);
+      sx = mfma_h(kl, qh[dk], sx);
+    }
+    // Lane holds keys 32 block + 16 (e / 8) + 8 hf + e % 8 of query q0 + col (log2 units).
+    const int kb = (blk0 + it) * 32;
+    if (kb + 32 > p.LK) {
+#pragma unroll
+      for (int e = 0; e < 16; e++)
+        if (kb + 16 * (e >> 3) + 8 * hf + (e & 7) >= p.LK) { sh[e] = -INFINITY; sx[e] = 0.f; }
+    }
+    float t[16];
+    auto relative = [&]() {
+#pragma unroll
+      for (int e = 0; e < 16; e++) t[e] = __builtin_fmaf(sx[e], 1.0f / 2048.0f, sh[e] - mb);
+    };
+    auto top16 = [&]() {
+      const float a = fmaxf(fmaxf(t[0], t[1]), t[2]), c = fmaxf(fmaxf(t[3], t[4]), t[5]);
+      const float d = fmaxf(fmaxf(t[6], t[7]), t[8]), f = fmaxf(fmaxf(t[9], t[10]), t[11]);
+      const float g = fmaxf(fmaxf(t[12], t[13]), t[14]);
+      return fmaxf(fmaxf(fmaxf(a, c), fmaxf(d, f)), fmaxf(g, t[15]));
+    };
+    float sum;
+    auto probabilities = [&]() {
+      float q[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        t[e] = __builtin_amdgcn_exp2f(t[e]) * 256.0f;
+        q[e & 3] += t[e];
+      }
+      sum = (q[0] + q[1]) + (q[2] + q[3]);
+    };
+    relative();
+    probabilities();
+    if (__ballot(sum > 32768.f)) {   // a score above the base by up to 7 (the first block's: by 1e30)
+      const float old = mb;
+      mb = 0.f;
+      relative();   // the scores themselves
+      mb = fmaxf(old, split_halves_max(top16()));
+      const float alpha = exp2f(old - mb);
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) { oh[db][e] *= alpha; ol[db][e] *= alpha; ox[db][e] *= alpha; }
+      relative();
+      probabilities();
+    }
+    l += sum;
+    f16x8 ph[2], pl[2];
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      asm volatile("" : "+v"(t[e]));   // one fp32 value feeds both halves
+      const f16 hi = (f16)t[e];
+      ph[e >> 3][e & 7] = hi;
+      pl[e >> 3][e & 7] = (f16)(t[e] - (float)hi);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+      for (int db = 0; db < DB; db++) {
+        const f16x8 vh = frag(slot, 2 * NF + ks * DB + db), vl = frag(slot, 3 * NF + ks * DB + db);
+        oh[db] = mfma_h(vh, ph[ks], oh[db]);
+        ol[db] = mfma_h(vh, pl[ks], ol[db]);
+        ox[db] = mfma_h(vl, ph[ks], ox[db]);
+      }
+  }
+  l = split_halves_sum(l);
+  const int qo = q0 + col;
+  if (p.S > 1) {
+    f32x4* dst = reinterpret_cast<f32x4*>(p.part) + ((((int64_t)bh * nq + qt) * p.S + range) * 4 + wave) * ((D / 4 + 1) * 32);
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        f32x4 out;
+#pragma unroll
+        for (int r = 0; r < 4; r++) out[r] = oh[db][4 * j + r] + (ol[db][4 * j + r] + ox[db][4 * j + r] * (1.0f / 2048.0f));
+        dst[(db * 8 + 2 * j + hf) * 32 + col] = out;
+      }
+    if (hf == 0) dst[D / 4 * 32 + col] = (f32x4){mb, l, 0.f, 0.f};
+  } else if (qo < p.L) {
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    float* orow = p.o + (int64_t)b * p.os0 + (int64_t)h * p.os2 + (int64_t)qo * p.os1;
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        f32x4 out;
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          out[r] = (oh[db][4 * j + r] + (ol[db][4 * j + r] + ox[db][4 * j + r] * (1.0f / 2048.0f))) * inv;
+        *reinterpret_cast<f32x4*>(orow + db * 32 + j * 8 + 4 * hf) = out;
+      }
+  }
+}
+
+// One thread per (query, four dims): o = sum_r 2^(mb_r - M) O_r / sum_r 2^(mb_r - M) l_r, in range order.
+template <int D>
+__global__ __launch_bounds__(256) void attention_planes_merge_kernel(PlanesAttnParams p) {
+  touch_args(p);
+  constexpr int NC = D / 4;
+  const int nq = (p.L + 127) / 128, tile = blockIdx.x;   // (batch * head, query tile, wave), 32 queries
+  const int col = threadIdx.x & 31, c0 = threadIdx.x >> 5;
+  const int wave = tile & 3, qt = (tile >> 2) % nq, bh = (tile >> 2) / nq, b = bh / p.H, h = bh % p.H;
+  const int qo = qt * 128 + wave * 32 + col;
+  if (qo >= p.L) return;
+  const f32x4* src = reinterpret_cast<const f32x4*>(p.part) + (((int64_t)bh * nq + qt) * p.S * 4 + wave) * ((NC + 1) * 32);
+  const int64_t step = 4 * (NC + 1) * 32;   // range to range
+  float M = -INFINITY;
+  for (int r = 0; r < p.S; r++) M = fmaxf(M, src[r * step + NC * 32 + col][0]);
+  float den = 0.f;
+  f32x4 num[NC / 8];
+#pragma unroll
+  for (int i = 0; i < NC / 8; i++) num[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < p.S; r++) {
+    const f32x4 ml = src[r * step + NC * 32 + col];
+    const float w = exp2f(ml[0] - M);
+    den += w * ml[1];
+#pragma unroll
+    for (int i = 0; i < NC / 8; i++) num[i] += w * src[r * step + (c0 + 8 * i) * 32 + col];
+  }
+  const float inv = den > 0.f ? 1.0f / den : 0.f;
+  float* orow = p.o + (int64_t)b * p.os0 + (int64_t)h * p.os2 + (int64_t)qo * p.os1;
+#pragma unroll
+  for (int i = 0; i < NC / 8; i++) *reinterpret_cast<f32x4*>(orow + 4 * (c0 + 8 * i)) = num[i] * inv;
+}
+
 // ------------------------------------------------------------------ conv (one pass)
 // y = act(((W_h x_h + (W_h x_l + W_l x_h) 2^-11) + (bias + shift)) * scale + residual) in one
 // launch: the FP32 input is read, prepared (GroupNorm affine, SiLU, nearest-2x upsampling,
@@ -1283,6 +1540,69 @@ int conv3d_exact(const ldx_conv3d_args* a, void* stream) {
   return launch_exact<3, 1, 2, 4, 4, 4, 1>(p, nb, st);
 }
 
+// Whether an FP32 attention call's rows allow 16-byte accesses and its head width the matrix units.
+static bool split_eligible(const ldx_attention_args* a) {
+  if (a->head_dim != 32 && a->head_dim != 64) return false;
+  const int64_t* ss[4] = {a->q_stride, a->k_stride, a->v_stride, a->o_stride};
+  const void* ps[4] = {a->q, a->k, a->v, a->o};
+  for (int i = 0; i < 4; i++) {
+    if ((uintptr_t)ps[i] % 16) return false;
+    for (int j = 0; j < 3; j++)
+      if (ss[i][j] % 4) return false;
+  }
+  return true;
+}
+
+// Key ranges of the three-launch form (0: the one-launch kernel, for fewer than 20 key blocks,
+// where two more launches cost more than they give: 512 tokens x 2 heads 24 us against 28, 1,000 x 4
+// 43 against 28, 2,500 x 2 99 against 29, 200 queries x 20,000 keys 717 against 47): the least
+// ceil(workgroups / CUs) x (blocks per range + 3), a CU counted as no emptier than two
+// workgroups (it needs that many waves to overlap one's VALU with another's MFMAs).
+static int planes_ranges(const ldx_attention_args* a) {
+  const int64_t nblk = ((int64_t)a->kv_len + 31) / 32, n = ((int64_t)a->q_len + 127) / 128 * a->batch * a->heads;
+  if (nblk < 20 || n > (1 << 20) || (int64_t)a->batch * a->heads > 65535 || nblk > (1 << 24)) return 0;
+  int best = 1;
+  int64_t least = INT64_MAX;
+  for (int s = 1; s <= 16 && s <= nblk; s++) {
+    const int64_t k = (n * s + 255) / 256, per = (nblk + s - 1) / s;
+    const int64_t cost = (k > 2 ? k : 2) * (per + 3);
+    if (cost < least) { least = cost; best = s; }
+  }
+  const int64_t per = (nblk + best - 1) / best;
+  return (int)((nblk + per - 1) / per);   // no empty range
+}
+
+size_t attention_f32_workspace_bytes(const ldx_attention_args* a) {
+  if (!a || a->batch < 1 || a->heads < 1 || a->q_len < 1 || a->kv_len < 1 || a->mask || !split_eligible(a)) return 0;
+  const int S = planes_ranges(a), D = a->head_dim;
+  if (!S) return 0;
+  const int64_t bh = (int64_t)a->batch * a->heads, nblk = ((int64_t)a->kv_len + 31) / 32;
+  const int64_t planes = bh * nblk * D * 32 * 8, part = S > 1 ? bh * ((a->q_len + 127) / 128) * S * 4 * (D / 4 + 1) * 32 * 16 : 0;
+  return (size_t)(planes + part);
+}
+
+template <int D>
+static int launch_planes(const ldx_attention_args* a, int S, hipStream_t st) {
+  PlanesAttnParams p{};
+  p.B = a->batch; p.H = a->heads; p.L = a->q_len; p.LK = a->kv_len;
+  p.nblk = (a->kv_len + 31) / 32; p.S = S; p.per = (p.nblk + S - 1) / S;
+  p.q = (const float*)a->q; p.qs0 = a->q_stride[0]; p.qs1 = a->q_stride[1]; p.qs2 = a->q_stride[2];
+  p.k = (const float*)a->k; p.ks0 = a->k_stride[0]; p.ks1 = a->k_stride[1]; p.ks2 = a->k_stride[2];
+  p.v = (const float*)a->v; p.vs0 = a->v_stride[0]; p.vs1 = a->v_stride[1]; p.vs2 = a->v_stride[2];
+  p.o = (float*)a->o; p.os0 = a->o_stride[0]; p.os1 = a->o_stride[1]; p.os2 = a->o_stride[2];
+  p.c = a->scale * 1.44269504088896341f;
+  const int64_t bh = (int64_t)p.B * p.H, nq = (p.L + 127) / 128;
+  p.planes = (f16*)a->workspace;
+  p.part = (float*)((char*)a->workspace + bh * p.nblk * D * 32 * 8);
+  hipLaunchKernelGGL(split_kv_kernel<D>, dim3((unsigned)p.nblk, (unsigned)bh), dim3(256), 0, st, p);
+  if (int rc = check_launch("attention (fp32, planes)")) return rc;
+  hipLaunchKernelGGL(attention_planes_kernel<D>, dim3((unsigned)(nq * bh * S)), dim3(256), 0, st, p);
+  if (int rc = check_launch("attention (fp32)")) return rc;
+  if (S == 1) return LDX_OK;
+  hipLaunchKernelGGL(attention_planes_merge_kernel<D>, dim3((unsigned)(nq * bh * 4)), dim3(256), 0, st, p);
+  return check_launch("attention (fp32, merge)");
+}
+
 int attention_f32(const ldx_attention_args* a, void* stream) {
   if (!a || !a->q || !a->k || !a->v || !a->o) return fail("attention (fp32): null pointer");
   if (a->batch < 1 || a->heads < 1 || a->q_len < 1 || a->kv_len < 1) return fail("attention (fp32): empty input");
@@ -1294,21 +1614,18 @@ int attention_f32(const ldx_attention_args* a, void* stream) {
   // (LDX_ATTN_F32=valu keeps the VALU kernel, for comparison); width 16 and other
   // layouts on the VALU kernel.
   const int D = a->head_dim;
-  bool aligned = true;
-  const int64_t* ss[4] = {a->q_stride, a->k_stride, a->v_stride, a->o_stride};
-  const void* ps[4] = {a->q, a->k, a->v, a->o};
-  for (int i = 0; i < 4; i++) {
-    if ((uintptr_t)ps[i] % 16) aligned = false;
-    for (int j = 0; j < 3; j++)
-      if (ss[i][j] % 4) aligned = false;
-  }
   const char* env = getenv("LDX_ATTN_F32");
-  if ((D == 32 || D == 64) && aligned && !(env && strcmp(env, "valu") == 0)) {
+  if (split_eligible(a) && !(env && strcmp(env, "valu") == 0)) {
     // In-tile offsets are 32-bit: 32 key rows of K and of V.
-    for (int i = 1; i < 3; i++)
-      if (ss[i][1] < 0 || ss[i][1] > (1 << 24)) return fail("attention (fp32): key stride out of range");
+    for (const int64_t ks : {a->k_stride[1], a->v_stride[1]})
+      if (ks < 0 || ks > (1 << 24)) return fail("attention (fp32): key stride out of range");
     const int64_t n = (int64_t)((a->q_len + 127) / 128) * a->heads * a->batch;
     if (n > 0x7fffffff) return fail("attention (fp32): grid too large");
+    const size_t need = attention_f32_workspace_bytes(a);
+    if (need && a->workspace && a->workspace_bytes >= need && al16(a->workspace)) {
+      const int S = planes_ranges(a);
+      return D == 32 ? launch_planes<32>(a, S, st) : launch_planes<64>(a, S, st);
+    }
     SplitAttnParams sp{};
     sp.B = a->batch; sp.H = a->heads; sp.L = a->q_len; sp.LK = a->kv_len;
     sp.q = (const float*)a->q; sp.qs0 = a->q_stride[0]; sp.qs1 = a->q_stride[1]; sp.qs2 = a->q_stride[2];

@@ -12,6 +12,7 @@ FP32 UNet with cross attention) and ``vq_float32`` (the FP32 decoder, quantized 
 
 from __future__ import annotations
 
+import ctypes
 import json
 
 import numpy as np
@@ -306,6 +307,40 @@ def test_fp32_attention_lmnet_length(pkg, dev) -> None:
     got = host(o)[:, :, rows]
     want = oatt.attention(q[:, :, rows].astype(np.float64), k.astype(np.float64), v.astype(np.float64), 32 ** -0.5)
     np.testing.assert_allclose(got, want, rtol=0, atol=2e-5)
+
+
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize(("batch", "heads", "lq", "lk"), [
+    (1, 1, 1, 609),       # one query, a last block of one key, as many key ranges as it takes
+    (2, 2, 129, 640),     # a query tile of one row, whole key blocks
+    (1, 3, 128, 1311),    # ranges of unequal length
+    (1, 1, 40000, 615),   # enough query tiles for one range: no merge
+])
+def test_fp32_attention_key_ranges(pkg, dev, d, batch, heads, lq, lk) -> None:
+    """The three-launch form (at least 20 key blocks) on head-interleaved views of one fused
+    projection, with scores that rise along the keys (the exponent base moves in every range)
+    and one query whose scores lie 80 below the others', against float64; also without the
+    workspace (the one-launch kernel), through the C ABI."""
+    rng = np.random.default_rng(lq + lk + d)
+    f = heads * d
+    q = rng.normal(size=(batch, lq, f)).astype(np.float32)
+    kv = rng.normal(size=(batch, lk, 2 * f)).astype(np.float32)
+    kv[..., :f] *= np.linspace(0.2, 4, lk, dtype=np.float32)[None, :, None]
+    q[:, 0] *= 8
+    qd, kvd = dev32(q, dev), dev32(kv, dev)
+    o = pkg.ops.flash_attention(qd, kvd[..., :f], kvd[..., f:], heads=heads, scale=d ** -0.5)
+    o2 = torch.empty_like(o)
+    a = pkg.ops._attn_args(qd.unflatten(2, (heads, d)), kvd[..., :f].unflatten(2, (heads, d)),
+                           kvd[..., f:].unflatten(2, (heads, d)), o2.unflatten(2, (heads, d)), d ** -0.5, None)
+    assert a.workspace_bytes > 0
+    a.workspace, a.workspace_bytes = None, 0
+    assert pkg._lib.lib.ldx_attention(ctypes.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    rows = np.unique(np.concatenate([[0], rng.integers(0, lq, 64), [lq - 1]]))
+    split = lambda t: t.astype(np.float64).reshape(batch, -1, heads, d).transpose(0, 2, 1, 3)  # noqa: E731
+    want = oatt.attention(split(q[:, rows]), split(kv[..., :f]), split(kv[..., f:]), d ** -0.5)
+    for got in (o, o2):
+        np.testing.assert_allclose(split(host(got[:, rows])), want, rtol=0, atol=2e-5)
 
 
 @pytest.mark.parametrize("d", [32, 64])
