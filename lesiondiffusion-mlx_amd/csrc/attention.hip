@@ -891,6 +891,188 @@ static int launch_attn(const AttnParams& p, hipStream_t st) {
   return check_launch("attention");
 }
 
+// Head widths 32 and 64 with enough 128-query tiles to fill the chip, no mask: a workgroup's
+// four waves own 4 x 32 queries and share 64-key stages of K and V, moved global->LDS by DMA
+// three deep (one barrier per 64 keys). The DMA lays K down in MFMA fragment order (each lane
+// picks its source address), so a K fragment is one lane-linear 16-byte read; V stays key-major
+// for the transposing reads (D = 64: the 64-byte halves of rows 2, 3 mod 4 swapped, so that
+// eight rows' reads meet all banks). Probabilities are formed against the current base with no
+// block maximum and the base moves only where a lane's 16 sum past 16 * 2^8, as in
+// attention_pipe_kernel's whole blocks. Against the register-staged attention_kernel<D, 1>:
+// no tile traffic through VGPRs (128 of them at D = 32: four waves per SIMD), 56 instead of
+// about 90 VALU operations per 32 x 32 block; bound by those (16 exp2 at a quarter rate).
+// 6,400 tokens x 16 heads of 32: 224 -> 155 us, 541 TFLOP/s (800 workgroups: four on some CUs
+// where the mean is 3.1).
+template <int D>
+__global__ __launch_bounds__(256, D == 32 ? 4 : 3) void attention_tile_kernel(AttnParams p) {
+  touch_args(p);
+  constexpr int DK = D / 16, DB = D / 32, KG = D / 8;
+  constexpr int SUB = 2 * 32 * D;             // elements of a 32-key sub-block: K fragments, then V rows
+  constexpr int RPD = 512 / D;                // V rows per DMA instruction
+  __shared__ __attribute__((aligned(16))) E smem[3 * 2 * SUB];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hf = lane >> 5, col = lane & 31;
+  int wg;   // query tiles of one head contiguous per XCD (one L2)
+  {
+    const int n = gridDim.x, l = blockIdx.x, per = n >> 3, rem = n & 7, x = l & 7, k = l >> 3;
+    wg = x < rem ? x * (per + 1) + k : rem * (per + 1) + (x - rem) * per + k;
+  }
+  const int nqb = (p.L + 127) / 128;
+  const int qblk = wg % nqb, h = (wg / nqb) % p.H, b = wg / nqb / p.H;
+  const int q0 = qblk * 128 + wave * 32, qi = min(q0 + col, p.L - 1);
+  const E* qb_ = p.q + (int64_t)b * p.qs0 + (int64_t)h * p.qs2;
+  E8 qf[DK];
+#pragma unroll
+  for (int dk = 0; dk < DK; dk++) qf[dk] = *reinterpret_cast<const E8*>(qb_ + (int64_t)qi * p.qs1 + dk * 16 + 8 * hf);
+#pragma unroll
+  for (int dk = 0; dk < DK; dk++) pin_value(qf[dk]);   // landed: only the DMAs below are counted from here on
+
+  // Of each stage wave 0 copies sub-block 0's K, wave 1 its V, waves 2 and 3 sub-block 1's:
+  // DK instructions of a kilobyte each.
+  const bool isv = wave & 1;
+  const E* src = isv ? p.v + (int64_t)b * p.vs0 + (int64_t)h * p.vs2 : p.k + (int64_t)b * p.ks0 + (int64_t)h * p.ks2;
+  const int64_t rs1 = isv ? p.vs1 : p.ks1;
+  unsigned off[DK];
+#pragma unroll
+  for (int i = 0; i < DK; i++) {
+    const int vr = RPD * i + lane / KG, vc = lane % KG;
+    off[i] = isv ? (unsigned)(vr * p.vs1 + (D == 64 ? vc ^ (((vr >> 1) & 1) << 2) : vc) * 8) * 2u
+                 : (unsigned)(key_row(col) * p.ks1 + 16 * i + 8 * hf) * 2u;
+  }
+  const unsigned dst0 = lds_offset(smem) + (unsigned)((wave >> 1) * SUB + (isv ? SUB / 2 : 0)) * 2u;
+  auto issue = [&](int st) {   // rows past the sequence read zeros
+    const int kbase = st * 64 + 32 * (wave >> 1), rows = min(32, p.LK - kbase);
+    const i32x4 rs = dma_rsrc(rows > 0 ? src + (int64_t)kbase * rs1 : src,
+                              rows > 0 ? (unsigned)(((rows - 1) * rs1 + D) * 2) : 0u);
+#pragma unroll
+    for (int i = 0; i < DK; i++)
+      dma_buffer_b128(rs, off[i], 0, dst0 + (unsigned)((st % 3) * 2 * SUB * 2 + i * 1024));
+  };
+  // V^T fragments (transposing reads): row 8 (lane / 32) + (lane % 16) / 4 (+ 16 ks, + 4 for the
+  // second half), dims 16 ((lane / 16) % 2) + 4 (lane % 4) (+ 32 db).
+  const int vrow = 8 * hf + ((lane & 15) >> 2), vdim = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  unsigned va[DB];   // LDS byte addresses in slot 0, sub-block 0
+#pragma unroll
+  for (int db = 0; db < DB; db++)
+    va[db] = lds_offset(smem) + (unsigned)(SUB / 2 + vrow * D + vdim + 32 * (DB == 2 ? db ^ ((vrow >> 1) & 1) : db)) * 2u;
+  typedef __attribute__((address_space(3))) char lds_char;
+  auto read_v = [](lds_char* a, int k) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(a + k)); };
+
+  f32x16 o[DB];
+#pragma unroll
+  for (int i = 0; i < DB; i++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) o[i][e] = 0.f;
+  float m = 0.f, l = 0.f;
+  const int nst = (p.LK + 63) / 64;
+
+  auto scores = [&](const E* sb) {
+    f32x16 s = {};
+#pragma unroll
+    for (int dk = 0; dk < DK; dk++) s = mfma32x(*reinterpret_cast<const E8*>(sb + dk * 512 + lane * 8), qf[dk], s);
+    return s;
+  };
+  // O^T += V^T P^T for the sub-block `slot` bytes into the ring, with scores s.
+  auto attend = [&](unsigned slot, const f32x16& s, int kbase) {
+    f32x16 t;
+    auto relative = [&]() {
+#pragma unroll
+      for (int e = 0; e < 16; e++) t[e] = __builtin_fmaf(s[e], p.c, -m);
+      if (kbase + 32 > p.LK) {
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+          if (kbase + 16 * (e >> 3) + 8 * hf + (e & 7) >= p.LK) t[e] = -INFINITY;
+      }
+    };
+    float sum;
+    unsigned pk[8];
+    auto probs = [&]() {
+      float s0, s1;
+#pragma unroll
+      for (int e = 0; e < 16; e += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(t[e]), p1 = __builtin_amdgcn_exp2f(t[e + 1]);
+        pk[e >> 1] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){p0, p1}, E2));
+        s0 = e == 0 ? p0 : s0 + p0;
+        s1 = e == 0 ? p1 : s1 + p1;
+      }
+      sum = s0 + s1;
+    };
+    relative();
+    probs();
+    if (__builtin_expect(__ballot(!(sum <= 16.f * 256.f)) != 0, 0)) {   // (inf and NaN too)
+      const float top = halves_max(max16(t)), d = top > 8.f ? top : 0.f, alpha = __builtin_amdgcn_exp2f(-d);
+      m += d;
+      relative();
+      probs();
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) o[db][e] *= alpha;
+    }
+    l += sum;
+    const E8 pf[2] = {__builtin_bit_cast(E8, (u32x4){pk[0], pk[1], pk[2], pk[3]}),
+                      __builtin_bit_cast(E8, (u32x4){pk[4], pk[5], pk[6], pk[7]})};
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+      for (int db = 0; db < DB; db++) {
+        lds_char* v = (lds_char*)(uintptr_t)(va[db] + slot);
+        const s16x4 lo = read_v(v, ks * 32 * D), hi = read_v(v, ks * 32 * D + 8 * D);
+        o[db] = mfma32x(__builtin_bit_cast(E8, (s16x8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}), pf[ks],
+                        o[db]);
+      }
+  };
+
+  vmcnt_wait<0>();
+  issue(0);
+  if (nst > 1) issue(1);
+  for (int st = 0; st < nst; st++) {
+    // This wave's share of stage st has landed when at most stage st + 1's is outstanding; after
+    // the barrier so have the others', and stage st - 1's slot is free.
+    if (st + 1 < nst) vmcnt_wait<DK>();
+    else vmcnt_wait<0>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (st + 2 < nst) issue(st + 2);
+    const E* sb = smem + (st % 3) * 2 * SUB;
+    const unsigned slot = (unsigned)((st % 3) * 2 * SUB) * 2u;
+    const f32x16 s0 = scores(sb), s1 = scores(sb + SUB);
+    if (st == 0) {   // the base: the first sub-block's maximum
+      f32x16 t;
+#pragma unroll
+      for (int e = 0; e < 16; e++)
+        t[e] = 16 * (e >> 3) + 8 * hf + (e & 7) < p.LK ? __builtin_fmaf(s0[e], p.c, 0.f) : -INFINITY;
+      m = halves_max(max16(t));
+    }
+    attend(slot, s0, st * 64);
+    if (st * 64 + 32 < p.LK) attend(slot + SUB * 2, s1, st * 64 + 32);
+  }
+  l = halves_sum(l);
+  const int qo = q0 + col;
+  if (qo >= p.L) return;
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  E* orow = p.o + (int64_t)b * p.os0 + (int64_t)h * p.os2 + (int64_t)qo * p.os1;
+#pragma unroll
+  for (int db = 0; db < DB; db++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      E4 out;
+#pragma unroll
+      for (int r = 0; r < 4; r++) out[r] = (E)(o[db][j * 4 + r] * inv);
+      *reinterpret_cast<E4*>(orow + db * 32 + j * 8 + 4 * hf) = out;
+    }
+}
+
+template <int D>
+static int launch_attn_tile(const AttnParams& p, hipStream_t st) {
+  const int64_t n = (int64_t)((p.L + 127) / 128) * p.H * p.B;
+  if (n > 0x7fffffff) return fail("attention: grid too large");
+  hipLaunchKernelGGL(attention_tile_kernel<D>, dim3((unsigned)n), dim3(256), 0, st, p);
+  return check_launch("attention");
+}
+
 // Wide heads (D = 128, 256; the VQ decoder's single 256-wide head over 51,200 tokens): a
 // workgroup's 4 waves own 4 x 32 queries and share every K/V tile. Tiles move global->LDS
 // by DMA (rows of D halves, 16-byte chunk c of row r at chunk position c ^ (r mod D/8);
@@ -1303,7 +1485,7 @@ static int launch_attn_wide(AttnParams p, hipStream_t st) {
 }
 
 // The kernel family launch_d picks: 1 / 4 / 8 (register-staged, key split), -4 / -8
-// (pipelined DMA key split) or -1 (wide heads).
+// (pipelined DMA key split), -3 (shared DMA tiles) or -1 (wide heads).
 template <int D>
 static int attn_split(const AttnParams& p) {
   // Key-split workgroups when 128-query workgroups would leave most CUs idle: for long
@@ -1313,6 +1495,10 @@ static int attn_split(const AttnParams& p) {
   int split = 1;
   if (const char* env = getenv("LDX_ATTN_SPLIT")) split = atoi(env);
   else if (D == 128 && wgs >= 256) split = -1;   // enough 128-query workgroups to fill the CUs
+  // From one and a half 128-query workgroups per CU on, shared tiles (us, the next choice below /
+  // attention_tile_kernel: 6,400 tokens x 16 heads of 32 224 / 155, 4,096 x 16 of 32 83 / 63, 6,400 x
+  // 8 of 64 147 / 123, 2,000 x 24 of 64 47.7 / 43; 336 workgroups 43 / 46, 208 25 / 26).
+  else if ((D == 32 || D == 64) && !p.mask && wgs >= 384 && p.LK >= 512) split = -3;
   else if (D <= 128 && wgs < 512 && p.LK > 64)
     split = (D == 32 || D == 64) && p.LK >= 512 ? -4 : (D <= 64 && p.LK >= 512) ? 8 : 4;
   return split;
@@ -1341,9 +1527,10 @@ template <int D>
 static int launch_d(const AttnParams& p, hipStream_t st) {
   const int split = attn_split<D>(p);
   if constexpr (D == 32 || D == 64) {
+    if (split == -3 && !p.mask) return launch_attn_tile<D>(p, st);
     // Long key sequences: the DMA-fed, software-pipelined four-way key split
     // (LDX_ATTN_SPLIT=-4 selects it for any length, -42 with query-block pairs; -8 the
-    // eight-way split).
+    // eight-way split, -3 the shared tiles).
     if (split == -4 && !getenv("LDX_ATTN_SPLIT") && pipe_pairs(p)) return launch_attn_pipe<D, 4, 2>(p, st);
     if (split == -4) return launch_attn_pipe<D, 4>(p, st);
     if (split == -42) return launch_attn_pipe<D, 4, 2>(p, st);

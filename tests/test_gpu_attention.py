@@ -123,6 +123,39 @@ def test_attention_key_split_variants_match_float64(pkg, dev, monkeypatch, split
     assert_fp16_bar(act, exp)
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize(("b", "heads", "lq", "lk", "forced"), [
+    (1, 2, 129, 1, True),      # one key, one query past a tile
+    (2, 3, 31, 33, True),      # the second sub-block of one key
+    (1, 2, 128, 96, True),     # whole sub-blocks, an odd number of them
+    (1, 1, 200, 1000, True),   # the ring's slots several times over, a ragged end
+    (3, 16, 1000, 513, False),   # 384 tiles: the launcher's own choice
+])
+def test_attention_shared_tiles_match_float64(pkg, dev, monkeypatch, dtype, d, b, heads, lq, lk, forced) -> None:
+    """The kernel with shared DMA tiles (LDX_ATTN_SPLIT=-3) on head-interleaved views of one wider
+    tensor, with scores that rise along the keys (the base moves) and a query 8 times the others,
+    at the kernels' bounds (bf16: 2^3 times fp16's step)."""
+    if forced:
+        monkeypatch.setenv("LDX_ATTN_SPLIT", "-3")
+    else:
+        monkeypatch.delenv("LDX_ATTN_SPLIT", raising=False)
+    tt = getattr(torch, dtype)
+    rng = np.random.default_rng(lq + 3 * lk + d)
+    f = heads * d
+    q, kv = rng.normal(size=(b, lq, f)).astype(np.float32), rng.normal(size=(b, lk, 2 * f)).astype(np.float32)
+    kv[..., :f] *= np.linspace(0.2, 4, lk, dtype=np.float32)[None, :, None]
+    q[:, 0] *= 8
+    qd, kvd = torch.from_numpy(q).to(tt).to(dev), torch.from_numpy(kv).to(tt).to(dev)
+    out = pkg.ops.flash_attention(qd, kvd[..., :f], kvd[..., f:], heads=heads, scale=d ** -0.5)
+    torch.cuda.synchronize()
+    rows = np.unique(np.concatenate([[0], rng.integers(0, lq, 48), [lq - 1]]))
+    split = lambda t: t.double().cpu().numpy().reshape(b, -1, heads, d).transpose(0, 2, 1, 3)  # noqa: E731
+    exp = oatt.attention(split(qd[:, rows]), split(kvd[..., :f]), split(kvd[..., f:]), d ** -0.5)
+    tol = 2e-3 if dtype == "float16" else 1.6e-2
+    np.testing.assert_allclose(split(out[:, rows]), exp, rtol=tol, atol=tol)
+
+
 @pytest.mark.parametrize("shares", ["1,1,1,1", "5,1,3,2", "16,1,1,1"])
 @pytest.mark.parametrize("split", ["-4", "-42"])
 @pytest.mark.parametrize(("b", "h", "lq", "lk", "d", "masked"), [
