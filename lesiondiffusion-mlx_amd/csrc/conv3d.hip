@@ -465,7 +465,9 @@ __global__ __launch_bounds__(256) void conv3d_kernel(ConvParams p) {
   const int kq = 8 * (lane >> 5) + kg * KSG * 16;
   const int ob0 = oblk * (BO / 32);
   // The epilogue's bias and shift, requested now so the main loop hides their latency.
-  const EpiConst ec = epi_const<FO>(p, lane, ob0 + wo * FO, b);
+  // (Three output blocks per wave finish as two and one: 96 channels are no power of two.)
+  constexpr int FE = FO == 3 ? 2 : FO;
+  const EpiConst ec = epi_const<FE>(p, lane, ob0 + wo * FO, b);
 
   // Per-lane B-operand (voxel) bases in the halo.
   int lbase[FV];
@@ -703,8 +705,17 @@ __global__ __launch_bounds__(256) void conv3d_kernel(ConvParams p) {
     __syncthreads();  // every wave is done with the halo and the weight rings
     stg = reinterpret_cast<float*>(smem) + w4 * 32 * EPW;
   }
-  conv_epilogue<FO, FV>(p, ec, acc, stg, lane, wv, b, sidx, pd, ph, pw, d0, h0, w0,
-                        (parity * p.nbr + brick) * (WV * FV) + wv * FV);
+  const int schunk = (parity * p.nbr + brick) * (WV * FV) + wv * FV;
+  if constexpr (FO == 3) {
+    f32x16 a01[2][FV], a2[1][FV];
+#pragma unroll
+    for (int fv = 0; fv < FV; fv++) { a01[0][fv] = acc[0][fv]; a01[1][fv] = acc[1][fv]; a2[0][fv] = acc[2][fv]; }
+    conv_epilogue<2, FV>(p, ec, a01, stg, lane, wv, b, sidx, pd, ph, pw, d0, h0, w0, schunk);
+    const EpiConst ec2 = epi_const<1>(p, lane, ob0 + wo * FO + 2, b);
+    conv_epilogue<1, FV>(p, ec2, a2, stg, lane, wv, b, sidx, pd, ph, pw, d0, h0, w0, schunk);
+  } else {
+    conv_epilogue<FO, FV>(p, ec, acc, stg, lane, wv, b, sidx, pd, ph, pw, d0, h0, w0, schunk);
+  }
 }
 
 // Pointwise conv / dense layer: a GEMM whose operands both come straight from global
@@ -1224,6 +1235,18 @@ static void pick_brick(const ConvParams& p, int BV, int s, int ks, int& TD, int&
     }
 }
 
+// Bricks of the 96-channel tile (256 voxels), whose halo beside the weight ring leaves two
+// workgroups per CU: the one with the fewest launched voxel slots, and those slots.
+static int64_t pick_brick96(const ConvParams& p, int& TD, int& TH, int& TW) {
+  static const int k[3][3] = {{4, 8, 8}, {8, 4, 8}, {4, 4, 16}};
+  int64_t best = INT64_MAX;
+  for (const auto& b : k) {
+    const int64_t slots = ceil_div64(p.RD, b[0]) * ceil_div64(p.RH, b[1]) * ceil_div64(p.RW, b[2]) * 256;
+    if (slots < best) { best = slots; TD = b[0]; TH = b[1]; TW = b[2]; }
+  }
+  return best;
+}
+
 template <int WO, int WV, int FO, int FV, int CC, int KSZ, bool VEC>
 static int launch(ConvParams& p, int grid_z, hipStream_t stream, size_t halo_bytes) {
   constexpr int BO = WO * FO * 32;
@@ -1264,7 +1287,10 @@ static int launch(ConvParams& p, int grid_z, hipStream_t stream, size_t halo_byt
   p.dv_nbh = make_udiv((unsigned)p.NBH);
   dim3 grid((unsigned)nwg);
   void (*kern)(ConvParams);
-  if constexpr (VEC) {
+  if constexpr (FO == 3) {   // (256-voxel bricks: their halos never fit the planned path's registers)
+    p.nh = 0;
+    kern = conv3d_kernel<WO, WV, FO, FV, CC, KSZ, true, false, 1>;
+  } else if constexpr (VEC) {
     kern = p.nh == 0   ? conv3d_kernel<WO, WV, FO, FV, CC, KSZ, true, false, 1>
            : tps > 1 ? conv3d_kernel<WO, WV, FO, FV, CC, KSZ, true, true, KSZ>
                      : conv3d_kernel<WO, WV, FO, FV, CC, KSZ, true, true, 1>;
@@ -1381,6 +1407,20 @@ static int plan_conv(const ldx_conv3d_args* a, ConvParams& p, Tile& t, size_t& l
   // over channel chunks then spreads the weights over twice the workgroups (measured:
   // 4x5x5, 256 -> 256 channels 13.4 -> 12.0 us).
   else t = {2, 2, 1, 1, vec && p.taps > 1 && p.C % 64 == 0 && rows > 256 ? 64 : 32};
+  // Output channels that 96-row tiles hold with less padding than 64-row ones (96, 288, ...), from
+  // one round of workgroups (two per CU) on, unless its fewer brick shapes waste the gain.
+  // us, 64 x 256 / 96 x 256 tiles, GroupNorm + SiLU + residual: 128x160x160 96->96 2241 / 1622
+  // (1,005 TFLOP/s), 64x80x80 96->96 280 / 214 and 288->288 1991 / 1635, 50x61x70 96->96 328 / 123 (the
+  // 64-row tile's brick of least waste has a long halo there), 36x60x62 115 / 97, 30x50x52 (below
+  // 512 workgroups) the same.
+  if (p.taps == 27 && p.stride == 1 && vec && p.O > 64 && (p.C1 == 0 || p.C0 % 32 == 0)) {
+    const int64_t o96 = (p.O + 95) / 96, o64 = (p.O + 63) / 64;
+    int bd, bh, bw, td, th, tw;
+    const int64_t s96 = pick_brick96(p, td, th, tw);
+    pick_brick(p, 256, 1, 3, bd, bh, bw);
+    const int64_t s64 = ceil_div64(p.RD, bd) * ceil_div64(p.RH, bh) * ceil_div64(p.RW, bw) * 256;
+    if (o96 * 96 < o64 * 64 && s96 * o96 * 96 <= s64 * o64 * 64 && s96 / 256 * o96 * p.B >= 512) t = {1, 4, 3, 2, 32};
+  }
   // LDX_CONV_TILE="WO,WV,FO,FV,CC" overrides the tile heuristic (tuning sweeps).
   bool forced = false;
   if (const char* env = getenv("LDX_CONV_TILE")) {
@@ -1401,7 +1441,8 @@ static int plan_conv(const ldx_conv3d_args* a, ConvParams& p, Tile& t, size_t& l
   const int s = p.stride;
   int TD = 1, TH = 1, TW = 1;
   for (;;) {
-    pick_brick(p, t.BV(), s, ks, TD, TH, TW);
+    if (t.FO == 3) pick_brick96(p, TD, TH, TW);
+    else pick_brick(p, t.BV(), s, ks, TD, TH, TW);
     p.TD = TD; p.TH = TH; p.TW = TW;
     p.HD = ks == 1 ? TD : (s == 2 ? 2 * TD + 1 : TD + 2);
     p.HH = ks == 1 ? TH : (s == 2 ? 2 * TH + 1 : TH + 2);
@@ -1660,6 +1701,9 @@ static int conv3d_run(const ldx_conv3d_args* a, float* stats, bool dry, int64_t*
   LDX_TILE(1, 4, 2, 1)
   LDX_TILE(2, 2, 2, 2)
   LDX_TILE(2, 2, 1, 1)
+  if (t.WO == 1 && t.WV == 4 && t.FO == 3 && t.FV == 2 && t.CC == 32 && vec && p.taps == 27)
+    rc = launch<1, 4, 3, 2, 32, 3, true>(p, grid_z, st, lds);
+  else
   return fail("conv3d: no kernel for tile");
 #undef LDX_TILE
   if (rc != LDX_OK || p.split == 1) return rc;

@@ -480,6 +480,42 @@ def test_conv_keeps_group_norm_moments(pkg, dev, shape, out_c, stride, upsample,
     check_moments(pkg, dev, y, groups=groups)
 
 
+@pytest.mark.parametrize(("shape", "c0", "out_c"), [
+    ((1, 32, 37, 60, 62), 32, 96),   # partial bricks on every axis
+    ((2, 40, 24, 45, 64), 32, 76),   # concat with a partial chunk, a partial channel group in the third block
+    ((1, 16, 32, 32, 80), 16, 288),  # three 96-channel tiles
+])
+def test_conv3d_ninety_six_channel_tile(pkg, dev, conv_path, shape, c0, out_c) -> None:
+    """The 96-channel tile (512 workgroups or more) through the whole prologue and epilogue, its
+    moments and three output planes against float64."""
+    if conv_path != "default":
+        pytest.skip("no other kernel takes these channel counts")
+    x, w, b = case(shape, out_c, 3, sum(shape))
+    rng = np.random.default_rng(out_c)
+    n, c = shape[:2]
+    aff = np.stack([rng.normal(size=(n, c)), rng.normal(size=(n, c)) * 0.3], -1).astype(np.float32)
+    res = rng.normal(size=(n, *shape[2:], out_c)).astype(np.float16)
+    xd = to_dev(ndhwc(x), dev)
+    y = pkg.ops.nax_conv3d(xd[..., :c0].contiguous(), pkg.ops.pack_weight(to_dev(w, dev)), to_dev(b, dev),
+                           x1=xd[..., c0:].contiguous() if c0 < c else None, affine=to_dev(aff, dev), silu=True,
+                           residual=to_dev(res, dev), moments="always" if out_c % 8 == 0 else False)
+    torch.cuda.synchronize()
+    if out_c % 32 == 0:
+        check_moments(pkg, dev, y, groups=32)
+    got = host(y)
+    d = shape[2]
+    prep = onm.silu(onm.apply_affine(x.astype(np.float64), aff.astype(np.float64)))
+    for z in (0, d // 2, d - 1):   # a plane from the planes it reads, zeros outside the volume
+        lo, hi = max(z - 1, 0), min(z + 2, d)
+        sl = np.zeros((n, c, 3, *shape[3:]))
+        sl[:, :, lo - z + 1:hi - z + 1] = prep[:, :, lo:hi]
+        exp = ocv.conv3d(sl, w.astype(np.float64), b.astype(np.float64))[:, :, 1] + res[:, z].transpose(0, 3, 1, 2)
+        mag = ocv.conv3d_magnitude(sl, w.astype(np.float64), b.astype(np.float64))[:, :, 1] + np.abs(
+            res[:, z].transpose(0, 3, 1, 2).astype(np.float64))
+        err = np.abs(got[:, z].transpose(0, 3, 1, 2) - exp)
+        assert np.all(err <= half_spacing(exp) + (ACCUMULATION_EPS + OPERAND_ROUNDING) * mag)
+
+
 def test_group_norm_of_a_concat_from_moments(pkg, dev) -> None:
     """The decoder's GroupNorm over concat([x, skip]) from both producers' moments, with
     groups that straddle the two tensors (C = 96 + 64, 32 groups of 5 channels would not be
