@@ -1217,8 +1217,12 @@ struct Tile {
 };
 
 static void pick_brick(const ConvParams& p, int BV, int s, int ks, int& TD, int& TH, int& TW) {
-  // Minimise launched voxel slots (partial-brick waste), then the halo volume.
-  int64_t best_slots = INT64_MAX, best_halo = INT64_MAX;
+  // Minimise launched voxel slots (partial-brick waste) plus a quarter of the halo voxels staged
+  // (what a halo voxel's staging costs beside a slot's MFMAs), then the halo volume. By slots
+  // alone ragged volumes got long bricks with halos of four voxels per output: us, before / now,
+  // 61x77x83 32->32 73 / 48, 50x61x70 96->32 141 / 68, 53x71x34 256->256 stride 2 400 / 333, upsampling
+  // 41x33x57 64->32 136 / 76; weights of 0.1 to 0.5 within 5 % of each other.
+  int64_t best_cost = INT64_MAX, best_halo = INT64_MAX;
   for (int td = 1; td <= BV; td *= 2)
     for (int th = 1; td * th <= BV; th *= 2) {
       const int tw = BV / (td * th);
@@ -1229,8 +1233,9 @@ static void pick_brick(const ConvParams& p, int BV, int s, int ks, int& TD, int&
       const int hh = ks == 1 ? th : (s == 2 ? 2 * th + 1 : th + 2);
       const int hw = ks == 1 ? tw : (s == 2 ? 2 * tw + 1 : tw + 2);
       const int64_t halo = (int64_t)hd * hh * hw;
-      if (slots < best_slots || (slots == best_slots && halo < best_halo)) {
-        best_slots = slots; best_halo = halo; TD = td; TH = th; TW = tw;
+      const int64_t cost = 4 * slots + nb * halo;
+      if (cost < best_cost || (cost == best_cost && halo < best_halo)) {
+        best_cost = cost; best_halo = halo; TD = td; TH = th; TW = tw;
       }
     }
 }
@@ -1462,6 +1467,7 @@ static int plan_conv(const ldx_conv3d_args* a, ConvParams& p, Tile& t, size_t& l
     const size_t wbytes = (size_t)WRING * (t.BO() / 32) * (t.CC / 16) * 1024;
     if (lds + wbytes <= (forced ? 160u * 1024 : 80u * 1024) || (t.CC == 32 && t.FV == 1)) break;
     if (t.CC == 64) t.CC = 32;
+    else if (t.WO == 2 && t.FV == 2) t = {1, 4, 2, 2, 32};   // (2 x 2 wave tiles have no one-column form)
     else t.FV = 1;
   }
   if (lds + (size_t)WRING * (t.BO() / 32) * (t.CC / 16) * 1024 > 160 * 1024)

@@ -516,6 +516,37 @@ def test_conv3d_ninety_six_channel_tile(pkg, dev, conv_path, shape, c0, out_c) -
         assert np.all(err <= half_spacing(exp) + (ACCUMULATION_EPS + OPERAND_ROUNDING) * mag)
 
 
+@pytest.mark.parametrize(("grid", "c", "out_c", "stride", "up"), [
+    ((41, 33, 57), 16, 96, 1, True),    # 128 x 128 tiles (a brick by slots alone left no kernel for its halo)
+    ((1, 1, 4099), 16, 96, 1, True),    # one long row: no 128-voxel brick's halo fits
+    ((29, 31, 33), 16, 64, 2, False),
+    ((61, 47, 83), 8, 32, 1, False),    # 32 x 256 tiles
+    ((3, 130, 5), 24, 40, 1, False),
+])
+def test_conv3d_ragged_volumes(pkg, dev, conv_path, grid, c, out_c, stride, up) -> None:
+    """Volumes that no brick divides: the first, a middle and the last output plane against
+    float64."""
+    if conv_path != "default":
+        pytest.skip("general kernel only")
+    x, w, b = case((1, c, *grid), out_c, 3, sum(grid))
+    xt, x64 = to_dev(ndhwc(x), dev), x.astype(np.float64)
+    pack = pkg.ops.pack_upsample_weight if up else pkg.ops.pack_weight
+    y = pkg.ops.nax_conv3d(xt, pack(to_dev(w, dev)), to_dev(b, dev), stride=stride, upsample=up)
+    torch.cuda.synchronize()
+    n = int(y.shape[1])
+    planes = sorted({0, n // 2, n - 1})
+    w64, b64 = w.astype(np.float64), b.astype(np.float64)
+    if up:
+        w64 = ocv.f16(ocv.fold_upsample_weight(w.astype(np.float32)).astype(np.float64))
+        run = lambda f, wt, bs: ocv.upsample_conv_folded_planes(f, grid[0], wt, bs, planes=planes)  # noqa: E731
+    else:
+        run = lambda f, wt, bs: ocv.conv3d_planes(f, grid[0], wt, bs, stride=stride, planes=planes)  # noqa: E731
+    exp = run(lambda i: x64[:, :, i], w64, b64)
+    mag = run(lambda i: np.abs(x64[:, :, i]), np.abs(w64), np.abs(b64))
+    err = np.abs(ncdhw(host(y[:, planes])) - exp)
+    assert np.all(err <= half_spacing(exp) + ACCUMULATION_EPS * mag)
+
+
 def test_group_norm_of_a_concat_from_moments(pkg, dev) -> None:
     """The decoder's GroupNorm over concat([x, skip]) from both producers' moments, with
     groups that straddle the two tensors (C = 96 + 64, 32 groups of 5 channels would not be
