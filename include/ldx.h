@@ -230,6 +230,15 @@ int ldx_group_norm_affine_moments_ws(const float* m0, int64_t chunks0, int32_t c
 int ldx_group_norm_affine_f32(const float* x0, int64_t x0_pitch, int32_t c0, const float* x1, int64_t x1_pitch,
                               int32_t c1, int32_t batch, int64_t voxels, int32_t groups, const float* gamma,
                               const float* beta, float eps, float* affine, void* stream);
+/* The same with a workspace of ldx_group_norm_f32_workspace_bytes (0 for tensors that one
+ * launch serves): large tensors then take two launches, voxel chunks over all channels and a
+ * merge of their moments. A NULL or smaller workspace runs the one launch. Same results within
+ * FP32 summation order. */
+size_t ldx_group_norm_f32_workspace_bytes(int32_t batch, int64_t voxels, int32_t channels, int32_t groups);
+int ldx_group_norm_affine_f32_ws(const float* x0, int64_t x0_pitch, int32_t c0, const float* x1, int64_t x1_pitch,
+                                 int32_t c1, int32_t batch, int64_t voxels, int32_t groups, const float* gamma,
+                                 const float* beta, float eps, float* affine, void* workspace,
+                                 size_t workspace_bytes, void* stream);
 int ldx_layer_norm_f32(const float* x, int64_t x_pitch, int64_t rows, int32_t features, const float* gamma,
                        const float* beta, float eps, float* y, int64_t y_pitch, void* stream);
 
