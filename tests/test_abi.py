@@ -237,3 +237,26 @@ def test_network_rejects_bf16_at_construction(pkg) -> None:
         pkg.layers.SourceLayers({}, device="cpu", dtype=torch.bfloat16)
     with pytest.raises(ValueError, match="network dtype"):
         pkg.unet.LdmUnet({}, None, device="cpu", dtype=torch.bfloat16)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1, 8), (2, 1, 1, 1, 8), (1, 3, 1, 1, 8), (2, 3, 4, 5, 1), (2, 1, 4, 1, 6)])
+def test_voxel_pitch_and_head_views(pkg, shape) -> None:
+    """Contiguous tensors, channel slices and refused orders of ``voxel_pitch``; the head view of
+    interleaved projections is torch's own ``unflatten``."""
+    import torch
+
+    c = shape[-1]
+    assert pkg.ops.voxel_pitch(torch.empty(shape)) == c
+    wide = torch.empty(*shape[:-1], c + 4)
+    assert pkg.ops.voxel_pitch(wide[..., :c]) == (c + 4 if max(shape[:-1]) > 1 else c)
+    if c > 1:
+        with pytest.raises(ValueError, match="contiguous"):
+            pkg.ops.voxel_pitch(torch.empty(*shape[:-1], 2 * c)[..., ::2])
+    if shape[0] > 1 and shape[1] > 1:
+        with pytest.raises(ValueError, match="evenly spaced"):
+            pkg.ops.voxel_pitch(torch.empty(shape[0], 2 * shape[1], *shape[2:])[:, ::2])
+    for t in (torch.empty(shape[0], 7, 24), torch.empty(shape[0], 7, 72)[..., 24:48], torch.empty(2, 9, 24)[:, :7]):
+        view = t.unflatten(2, (3, 8))
+        assert pkg.ops._interleaved(t, "q", 8) == (view.data_ptr(), view.stride()[:3])
+    with pytest.raises(ValueError, match="head_dim must be contiguous"):
+        pkg.ops._interleaved(torch.empty(1, 24, 7).transpose(1, 2), "q", 8)

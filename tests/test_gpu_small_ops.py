@@ -200,3 +200,11 @@ def test_ddim_step_kernels_match_oracle(pkg, dev) -> None:
                              float(c["sigmas"][idx]), float(c["sqrt_one_minus"][idx]), z["noise"][it])
         got = x.cpu().numpy().reshape(1, 2, 2, 2, 4).transpose(0, 4, 1, 2, 3)
         np.testing.assert_allclose(got, xs, rtol=1e-5, atol=1e-5)
+
+
+def test_ops_launch_on_the_current_stream(pkg, dev) -> None:
+    assert pkg.ops._stream() == torch.cuda.current_stream().cuda_stream
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        assert pkg.ops._stream() == s.cuda_stream
+    assert pkg.ops._stream() == torch.cuda.current_stream().cuda_stream
