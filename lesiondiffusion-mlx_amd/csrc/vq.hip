@@ -17,6 +17,7 @@
 #include "common.h"
 
 #include <cmath>
+#include <type_traits>
 
 // Every rounding point above is explicit; no multiply-add may be fused behind the code's back
 // (the reference compiles its search with contraction off as well).
@@ -58,6 +59,23 @@ __device__ __forceinline__ T vq_distance(T zn, T cn, float dot) {
   return (T)(summed - doubled);
 }
 
+// Distance of code `code` to the position with components zs and squared norm zns.
+template <typename T>
+__device__ __forceinline__ T code_distance(const float (&zs)[4], T zns, const T* __restrict__ codebook,
+                                           const T* __restrict__ cb_norm, int code) {
+  const T* e = codebook + (int64_t)code * 4;
+  float dot = zs[0] * (float)e[0];
+  dot = __builtin_fmaf(zs[1], (float)e[1], dot);
+  dot = __builtin_fmaf(zs[2], (float)e[2], dot);
+  dot = __builtin_fmaf(zs[3], (float)e[3], dot);
+  asm volatile("" : "+v"(dot));   // an fp32 value: not fused with its rounding to fp16 (v_fma_mixlo)
+  return vq_distance<T>(zns, cb_norm[code], dot);
+}
+
+__device__ __forceinline__ float lane_f(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
 // The smallest of three, a NaN if one of them is (v_min3_f32 would drop it).
 __device__ __forceinline__ float min3_nan(float a, float b, float c) {
   float r;
@@ -78,6 +96,29 @@ __device__ __forceinline__ bool vq_chunk_better(float da, int ca, float db, int 
   return da < db || (da == db && ca < cb);
 }
 
+// The least of 32 MFMA results (none a NaN that matters: such positions are scanned).
+__device__ __forceinline__ float minimum16(f32x16 a, f32x16 b) {
+  float m[2] = {a[0], b[0]};
+#pragma unroll
+  for (int i = 1; i < 16; i++) {
+    m[0] = __builtin_elementwise_minimum(m[0], a[i]);
+    m[1] = __builtin_elementwise_minimum(m[1], b[i]);
+  }
+  return __builtin_elementwise_minimum(m[0], m[1]);
+}
+
+// The least value over the wave's lanes (finite or +inf), in every lane.
+__device__ __forceinline__ float wave_min(float v) {
+  auto ror = [](float x, auto n) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + decltype(n)::value, 0xf, 0xf, false));
+  };
+  v = fminf(v, ror(v, std::integral_constant<int, 8>{}));
+  v = fminf(v, ror(v, std::integral_constant<int, 4>{}));
+  v = fminf(v, ror(v, std::integral_constant<int, 2>{}));
+  v = fminf(v, ror(v, std::integral_constant<int, 1>{}));
+  return fminf(fminf(lane_f(v, 0), lane_f(v, 16)), fminf(lane_f(v, 32), lane_f(v, 48)));
+}
+
 // First pass: the least distance of each position over every chunk of 64 codes and the first
 // chunk that has it, from MFMA tiles of 32 codes (rows) x 32 positions (columns; PG column
 // groups per wave). Second pass: that chunk alone, in order, for the index. The first pass costs
@@ -91,15 +132,13 @@ __device__ __forceinline__ bool vq_chunk_better(float da, int ca, float db, int 
 // code. SPLIT = 4: the waves share 32 positions and each scans a quarter of every stage; for
 // few positions (launch_vq_nearest4).
 template <typename T, int PG, int SPLIT>
-__global__ __launch_bounds__(VQ_THREADS, SPLIT == 1 ? 4 : 3) void vq_nearest4_kernel(
-    const T* __restrict__ z, const T* __restrict__ z_norm, const T* __restrict__ codebook,
-    const T* __restrict__ cb_norm, int64_t P, int E, int32_t* __restrict__ indices, T* __restrict__ quantized) {
+__device__ __forceinline__ void exact_search(const T* __restrict__ z, const T* __restrict__ z_norm,
+                                             const T* __restrict__ codebook, const T* __restrict__ cb_norm, int64_t P,
+                                             int E, int32_t* __restrict__ indices, T* __restrict__ quantized,
+                                             float4* cb /* components 0, 2, 1, 3: lane half h reads (h, 2 + h) */,
+                                             T* cbn, float* s_best, int* s_chunk) {
   static_assert(SPLIT == 1 || (SPLIT == 4 && PG == 1), "whole scans, or quarters of one column group");
   constexpr bool HALF = sizeof(T) == 2;
-  __shared__ float4 cb[VQ_STAGE];   // components 0, 2, 1, 3: lane half h reads (h, 2 + h)
-  __shared__ __attribute__((aligned(16))) T cbn[VQ_STAGE];
-  __shared__ float s_best[SPLIT == 4 ? 128 : 1];
-  __shared__ int s_chunk[SPLIT == 4 ? 128 : 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = lane >> 5, col = lane & 31;
   const int64_t p0 = SPLIT == 1 ? ((int64_t)blockIdx.x * 4 + wave) * (32 * PG) : (int64_t)blockIdx.x * 32;
@@ -213,19 +252,11 @@ __global__ __launch_bounds__(VQ_THREADS, SPLIT == 1 ? 4 : 3) void vq_nearest4_ke
   }
   // Index of that distance in its chunk: a lane per code, one position at a time (64 codes are
   // one contiguous kilobyte; a lane per position gathers: 75 us more at 409,600 positions).
-  // A code's distance to the position whose components and |z|^2 are given.
   auto distance = [&](const float (&zs)[4], T zns, int code) {
-    const T* e = codebook + (int64_t)code * 4;
-    float dot = zs[0] * (float)e[0];
-    dot = __builtin_fmaf(zs[1], (float)e[1], dot);
-    dot = __builtin_fmaf(zs[2], (float)e[2], dot);
-    dot = __builtin_fmaf(zs[3], (float)e[3], dot);
-    asm volatile("" : "+v"(dot));   // an fp32 value: not fused with its rounding to fp16 (v_fma_mixlo)
-    return vq_distance<T>(zns, cb_norm[code], dot);
+    return code_distance<T>(zs, zns, codebook, cb_norm, code);
   };
 #pragma unroll
   for (int g = 0; g < PG; g++) {
-    auto lane_f = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
     const float znf = (float)zn[g];
     int found = 0x7fffffff;
 #pragma unroll 4
@@ -262,18 +293,251 @@ __global__ __launch_bounds__(VQ_THREADS, SPLIT == 1 ? 4 : 3) void vq_nearest4_ke
   }
 }
 
-// Fewer than 81,920 positions (320 workgroups of 256) leave waves idle: quarters of the scan
-// then. us, whole scans / quarters, 8,192 codes: 500 positions 134 / 33, 51,200 134 / 112,
-// 100,000 168 / 186, 409,600 447 / 667.
+template <typename T, int PG, int SPLIT>
+__global__ __launch_bounds__(VQ_THREADS, SPLIT == 1 ? 4 : 3) void vq_nearest4_kernel(
+    const T* __restrict__ z, const T* __restrict__ z_norm, const T* __restrict__ codebook,
+    const T* __restrict__ cb_norm, int64_t P, int E, int32_t* __restrict__ indices, T* __restrict__ quantized) {
+  __shared__ float4 cb[VQ_STAGE];
+  __shared__ __attribute__((aligned(16))) T cbn[VQ_STAGE];
+  __shared__ float s_best[SPLIT == 4 ? 128 : 1];
+  __shared__ int s_chunk[SPLIT == 4 ? 128 : 1];
+  exact_search<T, PG, SPLIT>(z, z_norm, codebook, cb_norm, P, E, indices, quantized, cb, cbn, s_best, s_chunk);
+}
+
+// 2^e of a nonzero value from its absolute bits; `zero` for 0. Whether it may be scaled.
+__device__ __forceinline__ int bits_exponent(unsigned bits, int zero) { return bits ? (int)(bits >> 23) - 127 : zero; }
+__device__ __forceinline__ bool bits_scalable(unsigned bits) {
+  return bits == 0 || (bits >= (unsigned)(127 - 40) << 23 && bits < (unsigned)(127 + 40) << 23);
+}
+__device__ __forceinline__ float pow2(int e) { return __int_as_float((127 + e) << 23); }
+
+// FP32 search from bounds. One v_mfma_f32_32x32x16_f16 per 32 codes x 32 positions gives
+// |e|^2 - 2 z.e (scaled by powers of two) to within E: z and e as hi + lo fp16 (zh.eh + zh.el +
+// zl.eh, twelve of the sixteen products), |e|^2 as three fp16 parts times a power of two. The
+// chosen code, whatever the rounding of the exact distances, lies in a 64-code chunk whose least
+// value is within 2 E of the least of all. Each lane keeps the two least chunks of its position
+// and the third's value: the first chunk, and the second where it is within 2 E, are searched with
+// the exact distances; a position whose third is too, or whose values cannot be scaled (zero and
+// 2^-40 to 2^40 can), gets an exact scan by its wave; a workgroup with more than VQ_SCANS of those
+// (crowded or repeated codes), or a codebook that cannot be scaled, runs the exact search.
+//   E, with zm and z1 the largest and the summed |z_c| of the position, em and nm the largest |e_c|
+//   and ||e|^2| of the codebook. The largest component is scaled to 2^10 or more, so that a split
+//   leaves 2^-12 (half the last bit of lo, and a part below 2^-14 counted as lost): 2^-22 of zm and of
+//   em, and lo.lo 2^-22 zm em, over four products and the factor 2; sixteen accumulations at 2^-23 of
+//   2.03 z1 em + 1.01 nm; the exact chain's roundings, 2^-24 each: 10 z1 em, 2 nm, 2 |zn|. Together
+//   em (3.9e-6 zm + 5e-6 z1) + 2.1e-6 nm + 1.2e-7 |zn|; rounded up below.
+// 0.6 VALU operations per pair (half a three-way minimum and the chunk's bookkeeping) beside 32
+// MFMA cycles per 1,024, against 2.5 and 128 of the exact pass. us, exact / bounds, normal data:
+// 409,600 positions x 8,192 codes 453 / 200, 409,600 x 1,024 92 / 61, 100,000 x 8,192 163 / 89. Bound
+// by latency in two rounds of workgroups: 1,600 of them, four per CU, 45 us for one alone. A codebook
+// of codes all within 1/8,192 of zero 297, normal codes repeated eightfold 608 (one position
+// in a workgroup's 256 to scan is 30 us; the scans of the kernel before the matrix units took 1,292).
+constexpr int VQ_BSTAGE = 1024;   // codes per stage: 32 bytes each
+constexpr int VQ_SCANS = 16;
+__global__ __launch_bounds__(VQ_THREADS, 4) void vq_nearest4_bounds_kernel(
+    const float* __restrict__ z, const float* __restrict__ z_norm, const float* __restrict__ codebook,
+    const float* __restrict__ cb_norm, int64_t P, int E, int32_t* __restrict__ indices,
+    float* __restrict__ quantized) {
+  __shared__ __attribute__((aligned(16))) char lds[VQ_STAGE * 20];
+  unsigned (*s_max)[2] = reinterpret_cast<unsigned (*)[2]>(lds);   // before the first stage
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = lane >> 5, col = lane & 31;
+  const int64_t p0 = ((int64_t)blockIdx.x * 4 + wave) * 64;
+  const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto load4 = [](const float* v) { return make_float4(v[0], v[1], v[2], v[3]); };
+  auto abs_bits = [](float v) { return (unsigned)__float_as_int(v) & 0x7fffffffu; };
+  auto max4 = [&](float4 v) { return max(max(abs_bits(v.x), abs_bits(v.y)), max(abs_bits(v.z), abs_bits(v.w))); };
+  // Largest component and squared norm of the codebook, as absolute bits (a NaN is the largest).
+  unsigned em = 0, nm = 0;
+#pragma unroll 8
+  for (int i = threadIdx.x; i < E; i += VQ_THREADS) {
+    em = max(em, max4(load4(codebook + (int64_t)i * 4)));
+    nm = max(nm, abs_bits(cb_norm[i]));
+  }
+#pragma unroll
+  for (int o = 32; o; o >>= 1) {
+    em = max(em, (unsigned)__shfl_xor((int)em, o, 64));
+    nm = max(nm, (unsigned)__shfl_xor((int)nm, o, 64));
+  }
+  if (lane == 0) { s_max[wave][0] = em; s_max[wave][1] = nm; }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; w++) { em = max(em, s_max[w][0]); nm = max(nm, s_max[w][1]); }
+  bool exact = !bits_scalable(em) || !bits_scalable(nm);
+  if (!exact) {
+    const int es = 10 - bits_exponent(em, 10), ns = 14 - bits_exponent(nm, 14);
+    const float e_scale = -2.f * pow2(es), n_scale = pow2(ns);
+    // This lane's position, and the B operands of the wave's two column groups.
+    const int64_t pos = p0 + lane;
+    const float4 zv = pos < P ? load4(z + pos * 4) : zero4;
+    float zn = 0.f;
+    if (pos < P) {
+      const float v[4] = {zv.x, zv.y, zv.z, zv.w};
+      zn = z_norm ? z_norm[pos] : squared_norm4<float>(v);
+    }
+    const unsigned zm = max4(zv);
+    f16x8 zb[2];
+#pragma unroll
+    for (int g = 0; g < 2; g++) {
+      const int64_t q = p0 + 32 * g + col;
+      const float4 v4 = q < P ? load4(z + q * 4) : zero4;
+      const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+      const unsigned m = max4(v4);
+      const int zs = bits_scalable(m) ? 10 - bits_exponent(m, 10) : 0;
+      const int bs = min(max(zs + es - ns, -14), 15);
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const float x = v[c] * pow2(zs);
+        const f16 hi = (f16)x, lo = (f16)(x - (float)hi);
+        zb[g][c] = half ? lo : hi;
+        zb[g][4 + c] = half ? (c < 3 ? (f16)pow2(bs) : (f16)0.f) : hi;
+      }
+    }
+    float m1 = INFINITY, m2 = INFINITY, m3 = INFINITY;
+    int c1 = 0, c2 = 0;
+    f16x8* frag = reinterpret_cast<f16x8*>(lds);   // [half][code]
+    const f32x16 zero = {};
+    for (int base = 0; base < E; base += VQ_BSTAGE) {
+      const int n = min(VQ_BSTAGE, E - base), nr = (n + VQ_CHUNK - 1) / VQ_CHUNK * VQ_CHUNK;
+      __syncthreads();   // the previous stage is no longer read
+      for (int i = threadIdx.x; i < nr; i += VQ_THREADS) {
+        f16x8 a = {}, b = {};
+        if (i < n) {
+          const float4 v4 = load4(codebook + (int64_t)(base + i) * 4);
+          const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+          const float x = cb_norm[base + i] * n_scale;
+          const f16 n0 = (f16)x, n1 = (f16)(x - (float)n0);
+          b[4] = n0; b[5] = n1; b[6] = (f16)(x - (float)n0 - (float)n1);
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            const float y = v[c] * e_scale;
+            a[c] = b[c] = (f16)y;
+            a[4 + c] = (f16)(y - (float)a[c]);
+          }
+        } else {
+          b[4] = (f16)INFINITY;   // past the last code
+        }
+        frag[i] = a;
+        frag[VQ_BSTAGE + i] = b;
+      }
+      __syncthreads();
+      for (int c0 = 0; c0 < nr; c0 += VQ_CHUNK) {
+        const f16x8 a0 = frag[half * VQ_BSTAGE + c0 + col], a1 = frag[half * VQ_BSTAGE + c0 + 32 + col];
+        float m[2];
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+          const f32x16 d0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, zb[g], zero, 0, 0, 0);
+          const f32x16 d1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, zb[g], zero, 0, 0, 0);
+          m[g] = minimum16(d0, d1);
+        }
+        // Lanes 0-31: the chunk's least value of column group 0; lanes 32-63: of group 1.
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(m[0]), __float_as_int(m[1]), false, false);
+        const float v = fminf(__int_as_float(sw[0]), __int_as_float(sw[1]));
+        const int id = (base + c0) / VQ_CHUNK;
+        m3 = __builtin_amdgcn_fmed3f(m2, v, m3);
+        c2 = v < m1 ? c1 : (v < m2 ? id : c2);
+        m2 = __builtin_amdgcn_fmed3f(m1, v, m2);
+        c1 = v < m1 ? id : c1;
+        m1 = fminf(m1, v);
+      }
+    }
+    const int zs = bits_scalable(zm) ? 10 - bits_exponent(zm, 10) : 0, bs = zs + es - ns;
+    const float zmf = __int_as_float((int)zm), emf = __int_as_float((int)em), nmf = __int_as_float((int)nm);
+    const float z1 = __builtin_fabsf(zv.x) + __builtin_fabsf(zv.y) + __builtin_fabsf(zv.z) + __builtin_fabsf(zv.w);
+    const float bound = emf * (4e-6f * zmf + 5.1e-6f * z1) + 2.2e-6f * nmf + 2e-7f * __builtin_fabsf(zn);
+    const float margin = 2.1f * bound * pow2(zs) * pow2(es);
+    const bool scaled = bits_scalable(zm) && bits_scalable(abs_bits(zn)) && bs >= -14 && bs <= 15;
+    const bool scan = pos < P && !(scaled && m3 > m1 + margin);
+    const bool two = !(m2 > m1 + margin);
+    const uint64_t scans = __ballot(scan), twos = __ballot(two);
+    int* s_count = reinterpret_cast<int*>(lds);
+    __syncthreads();   // the last stage is no longer read
+    if (lane == 0) s_count[wave] = __builtin_popcountll(scans);
+    __syncthreads();
+    exact = s_count[0] + s_count[1] + s_count[2] + s_count[3] > VQ_SCANS;
+    if (!exact) {
+      const float zl[4] = {zv.x, zv.y, zv.z, zv.w};
+      int found = 0;
+      // Searches codes k0 and up, a lane per code: the first of the least (d: its distance).
+      auto search = [&](int i, int k0, float& d) {
+        const float zi[4] = {lane_f(zl[0], i), lane_f(zl[1], i), lane_f(zl[2], i), lane_f(zl[3], i)};
+        const float v = code_distance<float>(zi, lane_f(zn, i), codebook, cb_norm, min(k0 + lane, E - 1));
+        d = wave_min(v);   // (past the last code: its distance again, at a higher lane)
+        return k0 + (int)__builtin_ctzll(__ballot(v == d));
+      };
+      float best = 0.f;
+#pragma unroll 8
+      for (int i = 0; i < 64; i++) {
+        float d;
+        const int code = search(i, __builtin_amdgcn_readlane(c1, i) * VQ_CHUNK, d);
+        if (lane == i) { found = code; best = d; }
+      }
+      for (uint64_t left = __ballot(two && !scan && pos < P); left; left &= left - 1) {
+        const int i = __builtin_ctzll(left), k0 = __builtin_amdgcn_readlane(c2, i) * VQ_CHUNK;
+        float d;
+        const int code = search(i, k0, d);
+        if (lane == i && (d < best || (d == best && code < found))) found = code;
+      }
+      for (uint64_t left = scans; left; left &= left - 1) {
+        const int i = __builtin_ctzll(left);
+        const float zi[4] = {lane_f(zl[0], i), lane_f(zl[1], i), lane_f(zl[2], i), lane_f(zl[3], i)};
+        const float zni = lane_f(zn, i);
+        float b = code_distance<float>(zi, zni, codebook, cb_norm, min(lane, E - 1));
+        int code = min(lane, E - 1);
+#pragma unroll 8
+        for (int k = lane + 64; k < E; k += 64) {
+          const float d = code_distance<float>(zi, zni, codebook, cb_norm, k);
+          const bool better = ((d != d) & (b == b)) | (d < b);   // codes ascend: the first stays
+          b = better ? d : b;
+          code = better ? k : code;
+        }
+#pragma unroll
+        for (int o = 32; o; o >>= 1) {
+          const float ob = __shfl_xor(b, o, 64);
+          const int oc = __shfl_xor(code, o, 64);
+          if (vq_chunk_better(ob, oc, b, code)) { b = ob; code = oc; }
+        }
+        if (lane == i) found = code;
+      }
+      if (pos < P) {
+        indices[pos] = found;
+        if (quantized) {
+          const float* e = codebook + (int64_t)found * 4;
+#pragma unroll
+          for (int c = 0; c < 4; c++) quantized[pos * 4 + c] = zl[c] + (e[c] - zl[c]);
+        }
+      }
+    }
+  }
+  if (exact) {
+    __syncthreads();
+    exact_search<float, 2, 1>(z, z_norm, codebook, cb_norm, P, E, indices, quantized, reinterpret_cast<float4*>(lds),
+                              reinterpret_cast<float*>(lds + VQ_STAGE * 16), nullptr, nullptr);
+  }
+}
+
+// Up to 24,576 positions the quarters' workgroups run at once (three per CU), whole scans leave
+// waves idle. FP32 above that: bounds. us, quarters / bounds, 8,192 codes: 500 positions 34 / 45,
+// 24,000 46 / 76, 28,000 77 / 76, 51,200 111 / 76, 100,000 163 / 89 (whole exact scans); 24,000 x
+// 1,024 14 / 17, 32,000 x 300 20 / 14. fp16, whose rounding would make the bounds wide: whole exact
+// scans from 81,920 positions (us, whole / quarters, 8,192 codes: 51,200 134 / 112, 100,000 168 /
+// 186, 409,600 447 / 667).
 template <typename T>
 static void launch_vq_nearest4(const T* z, const T* z_norm, const T* codebook, const T* cb_norm, int64_t P, int E,
                                int32_t* indices, T* quantized, hipStream_t st) {
-  if (P >= 81920)
-    hipLaunchKernelGGL((vq_nearest4_kernel<T, 2, 1>), dim3((unsigned)((P + 255) / 256)), dim3(VQ_THREADS), 0, st, z,
-                       z_norm, codebook, cb_norm, P, E, indices, quantized);
-  else
+  constexpr bool F32 = sizeof(T) == 4;
+  if (P <= (F32 ? 24576 : 81919)) {
     hipLaunchKernelGGL((vq_nearest4_kernel<T, 1, 4>), dim3((unsigned)((P + 31) / 32)), dim3(VQ_THREADS), 0, st, z,
                        z_norm, codebook, cb_norm, P, E, indices, quantized);
+    return;
+  }
+  const dim3 grid((unsigned)((P + 255) / 256));
+  if constexpr (F32)
+    hipLaunchKernelGGL(vq_nearest4_bounds_kernel, grid, dim3(VQ_THREADS), 0, st, z, z_norm, codebook, cb_norm, P, E,
+                       indices, quantized);
+  else
+    hipLaunchKernelGGL((vq_nearest4_kernel<T, 2, 1>), grid, dim3(VQ_THREADS), 0, st, z, z_norm, codebook, cb_norm, P, E,
+                       indices, quantized);
 }
 
 }  // namespace ldx

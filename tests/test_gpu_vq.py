@@ -135,3 +135,43 @@ def test_search_rejects_bad_arguments(pkg, dev) -> None:
                                   torch.zeros(5, dtype=torch.float16, device=dev))
     with pytest.raises(ValueError):
         pkg.ops.squared_norms4(torch.zeros((0, 4), dtype=torch.float16, device=dev))
+
+
+@pytest.mark.parametrize(("kind", "positions", "entries"), [
+    ("normal", 24576, 1025), ("normal", 24577, 1024), ("normal", 24833, 1), ("normal", 25000, 65),
+    ("crowded", 24600, 4133),      # many codes within the bounds' error of the least
+    ("repeated", 24600, 1500),     # every code eight times: the exact search of whole workgroups
+    ("lattice", 30001, 700),       # exact ties at midpoints
+    ("tiny", 24700, 2047), ("large", 24700, 2047),   # large: beyond the powers of two that scale
+    ("mixed", 24700, 3000), ("nan code", 24700, 300), ("infinite code", 24700, 300), ("zero codes", 24700, 129),
+])
+def test_search_from_bounds(pkg, dev, kind, positions, entries) -> None:
+    """FP32 above 24,576 positions, which searches only the chunks that fp16 bounds leave: every
+    index (of sampled rows, and of rows with NaN, infinite, zero and huge components) equals the
+    oracle's, for data on which the bounds decide little or nothing."""
+    rng = np.random.default_rng(positions + entries)
+    cb, flat = rng.normal(size=(entries, 4)), rng.normal(size=(positions, 4))
+    if kind == "crowded":
+        cb[entries // 3:] = rng.uniform(-1, 1, (entries - entries // 3, 4)) / entries
+    elif kind == "repeated":
+        cb = cb[rng.integers(0, entries // 8, entries)]
+    elif kind == "lattice":
+        cb, flat = rng.integers(-2, 3, cb.shape) * 1.0, rng.integers(-3, 4, flat.shape) / 2
+    elif kind == "tiny":
+        cb, flat = cb * 3e-3, flat * 1e-4
+    elif kind == "large":
+        cb, flat = cb * 1e7, flat * 1e7
+    elif kind == "mixed":
+        cb = cb * np.exp2(rng.integers(-12, 3, (entries, 1)))
+        flat = flat * np.exp2(rng.integers(-30, 30, (positions, 1)))
+    elif kind == "zero codes":
+        cb = cb * 0
+    cb, flat = cb.astype(np.float32), flat.astype(np.float32)
+    if kind.endswith("code"):
+        cb[entries // 3, 1] = np.nan if kind == "nan code" else np.inf
+    flat[3], flat[5, 2], flat[7, 1], flat[9] = 0, np.nan, -np.inf, 1e15
+    idx, _, _ = _search(pkg, dev, flat, cb, torch.float32)
+    rows = np.unique(np.concatenate([np.arange(16), positions - 1 - np.arange(16), rng.integers(0, positions, 400)]))
+    with np.errstate(invalid="ignore", over="ignore"):
+        want, _ = ovq.quantize4(flat[rows], cb, np.float32)
+    np.testing.assert_array_equal(idx[rows], want)
