@@ -328,7 +328,7 @@ __device__ __forceinline__ float pow2(int e) { return __int_as_float((127 + e) <
 //   em (3.9e-6 zm + 5e-6 z1) + 2.1e-6 nm + 1.2e-7 |zn|; rounded up below.
 // 0.6 VALU operations per pair (half a three-way minimum and the chunk's bookkeeping) beside 32
 // MFMA cycles per 1,024, against 2.5 and 128 of the exact pass. us, exact / bounds, normal data:
-// 409,600 positions x 8,192 codes 453 / 200, 409,600 x 1,024 92 / 61, 100,000 x 8,192 163 / 89. Bound
+// 409,600 positions x 8,192 codes 453 / 200, 409,600 x 1,024 92 / 61, 100,000 x 8,192 163 / 75. Bound
 // by latency in two rounds of workgroups: 1,600 of them, four per CU, 45 us for one alone. A codebook
 // of codes all within 1/8,192 of zero 297, normal codes repeated eightfold 608 (one position
 // in a workgroup's 256 to scan is 30 us; the scans of the kernel before the matrix units took 1,292).
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(VQ_THREADS, 4) void vq_nearest4_bounds_kernel(
 
 // Up to 24,576 positions the quarters' workgroups run at once (three per CU), whole scans leave
 // waves idle. FP32 above that: bounds. us, quarters / bounds, 8,192 codes: 500 positions 34 / 45,
-// 24,000 46 / 76, 28,000 77 / 76, 51,200 111 / 76, 100,000 163 / 89 (whole exact scans); 24,000 x
+// 24,000 46 / 76, 28,000 77 / 45, 51,200 111 / 75, 100,000 163 / 75 (whole exact scans); 24,000 x
 // 1,024 14 / 17, 32,000 x 300 20 / 14. fp16, whose rounding would make the bounds wide: whole exact
 // scans from 81,920 positions (us, whole / quarters, 8,192 codes: 51,200 134 / 112, 100,000 168 /
 // 186, 409,600 447 / 667).
