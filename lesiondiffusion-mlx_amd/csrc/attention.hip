@@ -97,6 +97,16 @@ __device__ __forceinline__ float max16(const f32x16& s) {
   const float t4 = fmaxf(fmaxf(s[12], s[13]), s[14]);
   return fmaxf(fmaxf(fmaxf(t0, t1), fmaxf(t2, t3)), fmaxf(t4, s[15]));
 }
+// The same maximum from IEEE 754-2019 maxima (NaN if one of the scores is): no canonicalisation
+// of MFMA results.
+__device__ __forceinline__ float maximum16(const f32x16& s) {
+  float t[5];
+#pragma unroll
+  for (int i = 0; i < 5; i++)
+    t[i] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(s[3 * i], s[3 * i + 1]), s[3 * i + 2]);
+  const float a = __builtin_elementwise_maximum(__builtin_elementwise_maximum(t[0], t[1]), t[2]);
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, t[3]), __builtin_elementwise_maximum(t[4], s[15]));
+}
 __device__ __forceinline__ float halves_sum(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
   return __int_as_float(r[0]) + __int_as_float(r[1]);
@@ -896,13 +906,11 @@ static int launch_attn(const AttnParams& p, hipStream_t st) {
 // three deep (one barrier per 64 keys). The DMA lays K down in MFMA fragment order (each lane
 // picks its source address), so a K fragment is one lane-linear 16-byte read; V stays key-major
 // for the transposing reads (D = 64: the 64-byte halves of rows 2, 3 mod 4 swapped, so that
-// eight rows' reads meet all banks). Probabilities are formed against the current base with no
-// block maximum and the base moves only where a lane's 16 sum past 16 * 2^8, as in
-// attention_pipe_kernel's whole blocks. Against the register-staged attention_kernel<D, 1>:
-// no tile traffic through VGPRs (128 of them at D = 32: four waves per SIMD), 56 instead of
-// about 90 VALU operations per 32 x 32 block; bound by those (16 exp2 at a quarter rate).
-// 6,400 tokens x 16 heads of 32: 224 -> 155 us, 541 TFLOP/s (800 workgroups: four on some CUs
-// where the mean is 3.1).
+// eight rows' reads meet all banks). The arithmetic is the register-staged attention_kernel<D, 1>'s
+// in its order (running maximum per 32 keys), so the outputs are its bits; against it, no tile
+// traffic through VGPRs (86 of them at D = 32: four waves per SIMD), three-input maxima, and the
+// rescale (with its exp2) skipped where no query's maximum moves. Bound by the VALU (16 exp2 at a
+// quarter rate per 32 x 32 block). 6,400 tokens x 16 heads of 32: 223 -> 182 us, 461 TFLOP/s.
 template <int D>
 __global__ __launch_bounds__(256, D == 32 ? 4 : 3) void attention_tile_kernel(AttnParams p) {
   touch_args(p);
@@ -963,7 +971,7 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 3) void attention_tile_kernel(At
   for (int i = 0; i < DB; i++)
 #pragma unroll
     for (int e = 0; e < 16; e++) o[i][e] = 0.f;
-  float m = 0.f, l = 0.f;
+  float m = -INFINITY, l = 0.f;
   const int nst = (p.LK + 63) / 64;
 
   auto scores = [&](const E* sb) {
@@ -972,45 +980,49 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 3) void attention_tile_kernel(At
     for (int dk = 0; dk < DK; dk++) s = mfma32x(*reinterpret_cast<const E8*>(sb + dk * 512 + lane * 8), qf[dk], s);
     return s;
   };
-  // O^T += V^T P^T for the sub-block `slot` bytes into the ring, with scores s.
-  auto attend = [&](unsigned slot, const f32x16& s, int kbase) {
-    f32x16 t;
-    auto relative = [&]() {
+  // O^T += V^T P^T for the sub-block `slot` bytes into the ring, with scores s: attention_kernel's
+  // block, operation for operation (alpha stays 1 where no query's maximum moved, as exp2(0) is).
+  auto attend = [&](unsigned slot, f32x16 s, int kbase) {
+    const bool whole = kbase + 32 <= p.LK;
+    float top;
+    if (whole) {
+      top = halves_max(maximum16(s)) * p.c;
+    } else {
+      top = -INFINITY;
 #pragma unroll
-      for (int e = 0; e < 16; e++) t[e] = __builtin_fmaf(s[e], p.c, -m);
-      if (kbase + 32 > p.LK) {
-#pragma unroll
-        for (int e = 0; e < 16; e++)
-          if (kbase + 16 * (e >> 3) + 8 * hf + (e & 7) >= p.LK) t[e] = -INFINITY;
+      for (int e = 0; e < 16; e++) {
+        const float t = s[e] * p.c;
+        s[e] = kbase + 16 * (e >> 3) + 8 * hf + (e & 7) < p.LK ? t : -INFINITY;
+        top = fmaxf(top, s[e]);
       }
-    };
-    float sum;
-    unsigned pk[8];
-    auto probs = [&]() {
-      float s0, s1;
-#pragma unroll
-      for (int e = 0; e < 16; e += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(t[e]), p1 = __builtin_amdgcn_exp2f(t[e + 1]);
-        pk[e >> 1] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){p0, p1}, E2));
-        s0 = e == 0 ? p0 : s0 + p0;
-        s1 = e == 0 ? p1 : s1 + p1;
-      }
-      sum = s0 + s1;
-    };
-    relative();
-    probs();
-    if (__builtin_expect(__ballot(!(sum <= 16.f * 256.f)) != 0, 0)) {   // (inf and NaN too)
-      const float top = halves_max(max16(t)), d = top > 8.f ? top : 0.f, alpha = __builtin_amdgcn_exp2f(-d);
-      m += d;
-      relative();
-      probs();
-      l *= alpha;
-#pragma unroll
-      for (int db = 0; db < DB; db++)
-#pragma unroll
-        for (int e = 0; e < 16; e++) o[db][e] *= alpha;
+      top = halves_max(top);
     }
-    l += sum;
+    float alpha = 1.f;
+    if (__ballot(top > m)) {
+      const float mn = fmaxf(m, top);
+      alpha = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+#pragma unroll
+      for (int db = 0; db < DB; db++) scale_in_place(o[db], alpha);
+    }
+    if (whole) {
+#pragma unroll
+      for (int e = 0; e < 16; e++) s[e] = __builtin_fmaf(s[e], p.c, -m);
+    } else {
+      const float base = m == -INFINITY ? 0.f : m;
+#pragma unroll
+      for (int e = 0; e < 16; e++) s[e] -= base;
+    }
+    float s0, s1;
+    unsigned pk[8];
+#pragma unroll
+    for (int e = 0; e < 16; e += 2) {
+      const float p0 = __builtin_amdgcn_exp2f(s[e]), p1 = __builtin_amdgcn_exp2f(s[e + 1]);
+      pk[e >> 1] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){p0, p1}, E2));
+      s0 = e == 0 ? p0 : s0 + p0;
+      s1 = e == 0 ? p1 : s1 + p1;
+    }
+    l = __builtin_fmaf(l, alpha, s0 + s1);
     const E8 pf[2] = {__builtin_bit_cast(E8, (u32x4){pk[0], pk[1], pk[2], pk[3]}),
                       __builtin_bit_cast(E8, (u32x4){pk[4], pk[5], pk[6], pk[7]})};
 #pragma unroll
@@ -1039,13 +1051,6 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 3) void attention_tile_kernel(At
     const E* sb = smem + (st % 3) * 2 * SUB;
     const unsigned slot = (unsigned)((st % 3) * 2 * SUB) * 2u;
     const f32x16 s0 = scores(sb), s1 = scores(sb + SUB);
-    if (st == 0) {   // the base: the first sub-block's maximum
-      f32x16 t;
-#pragma unroll
-      for (int e = 0; e < 16; e++)
-        t[e] = 16 * (e >> 3) + 8 * hf + (e & 7) < p.LK ? __builtin_fmaf(s0[e], p.c, 0.f) : -INFINITY;
-      m = halves_max(max16(t));
-    }
     attend(slot, s0, st * 64);
     if (st * 64 + 32 < p.LK) attend(slot + SUB * 2, s1, st * 64 + 32);
   }
@@ -1495,10 +1500,12 @@ static int attn_split(const AttnParams& p) {
   int split = 1;
   if (const char* env = getenv("LDX_ATTN_SPLIT")) split = atoi(env);
   else if (D == 128 && wgs >= 256) split = -1;   // enough 128-query workgroups to fill the CUs
-  // From one and a half 128-query workgroups per CU on, shared tiles (us, the next choice below /
-  // attention_tile_kernel: 6,400 tokens x 16 heads of 32 224 / 155, 4,096 x 16 of 32 83 / 63, 6,400 x
-  // 8 of 64 147 / 123, 2,000 x 24 of 64 47.7 / 43; 336 workgroups 43 / 46, 208 25 / 26).
-  else if ((D == 32 || D == 64) && !p.mask && wgs >= 384 && p.LK >= 512) split = -3;
+  // Where the key split ends (two 128-query workgroups per CU), shared tiles in place of
+  // attention_kernel<D, 1>, the same bits. us, attention_kernel / shared tiles: 6,400 tokens x 16
+  // heads of 32 223 / 182, 4,096 x 16 of 32 83 / 75 and of 64 104 / 100, 4,096 x 512 keys x 16 of 32
+  // 15 / 13.5. Fewer workgroups, key split / shared tiles: 2,000 x 24 of 64 46 / 53, 3,100 x 16 of 32
+  // 58 / 59, 6,400 x 8 of 64 145 / 146.
+  else if ((D == 32 || D == 64) && !p.mask && wgs >= 512 && p.LK >= 512) split = -3;
   else if (D <= 128 && wgs < 512 && p.LK > 64)
     split = (D == 32 || D == 64) && p.LK >= 512 ? -4 : (D <= 64 && p.LK >= 512) ? 8 : 4;
   return split;

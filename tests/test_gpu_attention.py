@@ -130,11 +130,11 @@ def test_attention_key_split_variants_match_float64(pkg, dev, monkeypatch, split
     (2, 3, 31, 33, True),      # the second sub-block of one key
     (1, 2, 128, 96, True),     # whole sub-blocks, an odd number of them
     (1, 1, 200, 1000, True),   # the ring's slots several times over, a ragged end
-    (3, 16, 1000, 513, False),   # 384 tiles: the launcher's own choice
+    (3, 16, 1400, 513, False),   # 528 tiles: the launcher's own choice
 ])
 def test_attention_shared_tiles_match_float64(pkg, dev, monkeypatch, dtype, d, b, heads, lq, lk, forced) -> None:
     """The kernel with shared DMA tiles (LDX_ATTN_SPLIT=-3) on head-interleaved views of one wider
-    tensor, with scores that rise along the keys (the base moves) and a query 8 times the others,
+    tensor, with scores that rise along the keys (the maximum moves) and a query 8 times the others,
     at the kernels' bounds (bf16: 2^3 times fp16's step)."""
     if forced:
         monkeypatch.setenv("LDX_ATTN_SPLIT", "-3")
@@ -154,6 +154,42 @@ def test_attention_shared_tiles_match_float64(pkg, dev, monkeypatch, dtype, d, b
     exp = oatt.attention(split(qd[:, rows]), split(kvd[..., :f]), split(kvd[..., f:]), d ** -0.5)
     tol = 2e-3 if dtype == "float16" else 1.6e-2
     np.testing.assert_allclose(split(out[:, rows]), exp, rtol=tol, atol=tol)
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize(("b", "heads", "lq", "lk", "forced"), [
+    (2, 3, 31, 33, True), (1, 2, 128, 96, True), (1, 1, 200, 1000, True), (1, 2, 130, 20, True),
+    (2, 8, 4096, 512, False),    # 512 tiles: the fewest the launcher gives the shared tiles
+    (1, 24, 2800, 1111, False),
+])
+def test_attention_shared_tiles_give_the_register_staged_bits(pkg, dev, monkeypatch, dtype, d, b, heads, lq, lk,
+                                                              forced) -> None:
+    """The shared DMA tiles against attention_kernel<D, 1> (LDX_ATTN_SPLIT=1), every output bit:
+    rising scores, a query 8 times the others, one whose scores are all equal, and an infinite
+    key component (its head's NaNs at the same places)."""
+    tt = getattr(torch, dtype)
+    rng = np.random.default_rng(7 * lq + lk + d)
+    f = heads * d
+    q, kv = rng.normal(size=(b, lq, f)).astype(np.float32), rng.normal(size=(b, lk, 2 * f)).astype(np.float32)
+    kv[..., :f] *= np.linspace(0.2, 4, lk, dtype=np.float32)[None, :, None]
+    q[:, 0] *= 8
+    q[:, 1] = 0
+    kv[-1, lk // 2, f - 1] = np.inf
+    qd, kvd = torch.from_numpy(q).to(tt).to(dev), torch.from_numpy(kv).to(tt).to(dev)
+    outs = []
+    for split in ("-3" if forced else None, "1"):
+        if split is None:
+            monkeypatch.delenv("LDX_ATTN_SPLIT", raising=False)
+        else:
+            monkeypatch.setenv("LDX_ATTN_SPLIT", split)
+        out = pkg.ops.flash_attention(qd, kvd[..., :f], kvd[..., f:], heads=heads, scale=d ** -0.5)
+        torch.cuda.synchronize()
+        outs.append(out.cpu())
+    nan = outs[1].isnan()
+    assert nan[-1, 1, (heads - 1) * d:].all() and not nan[..., :(heads - 1) * d].any()   # 0 * inf
+    assert torch.equal(outs[0].isnan(), nan)
+    assert torch.equal(outs[0].view(torch.int16)[~nan], outs[1].view(torch.int16)[~nan])
 
 
 @pytest.mark.parametrize("shares", ["1,1,1,1", "5,1,3,2", "16,1,1,1"])
