@@ -76,6 +76,12 @@ __device__ __forceinline__ float lane_f(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
+// Bits of the largest absolute component (a NaN is the largest).
+__device__ __forceinline__ unsigned max4_bits(float4 v) {
+  auto abs_bits = [](float x) { return __float_as_uint(x) & 0x7fffffffu; };
+  return max(max(abs_bits(v.x), abs_bits(v.y)), max(abs_bits(v.z), abs_bits(v.w)));
+}
+
 // The smallest of three, a NaN if one of them is (v_min3_f32 would drop it).
 __device__ __forceinline__ float min3_nan(float a, float b, float c) {
   float r;
@@ -119,11 +125,28 @@ __device__ __forceinline__ float wave_min(float v) {
   return fminf(fminf(lane_f(v, 0), lane_f(v, 16)), fminf(lane_f(v, 32), lane_f(v, 48)));
 }
 
+// The largest value over the wave's lanes, in every lane.
+__device__ __forceinline__ unsigned wave_max(unsigned v) {
+  auto ror = [](unsigned x, auto n) {
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x120 + decltype(n)::value, 0xf, 0xf, false);
+  };
+  v = max(v, ror(v, std::integral_constant<int, 8>{}));
+  v = max(v, ror(v, std::integral_constant<int, 4>{}));
+  v = max(v, ror(v, std::integral_constant<int, 2>{}));
+  v = max(v, ror(v, std::integral_constant<int, 1>{}));
+  auto row = [&](int l) { return (unsigned)__builtin_amdgcn_readlane((int)v, l); };
+  return max(max(row(0), row(16)), max(row(32), row(48)));
+}
+
 // First pass: the least distance of each position over every chunk of 64 codes and the first
 // chunk that has it, from MFMA tiles of 32 codes (rows) x 32 positions (columns; PG column
 // groups per wave). Second pass: that chunk alone, in order, for the index. The first pass costs
-// 2.5 VALU operations per pair (add, fused multiply-add with the exact 2 * dot in fp32, half a
-// three-way minimum) and 128 MFMA cycles per 1,024; a scan that carries the index costs nine.
+// 2.5 VALU operations per pair (add, fused multiply-add with 2 * dot in fp32, half a three-way
+// minimum) and 128 MFMA cycles per 1,024; a scan that carries the index costs nine. The fused form
+// is the reference's unless a finite dot's double overflows (its 2 * dot is then infinite), which
+// needs components with |z_c| |e_c| of 2^125: positions that could have such a dot (2^124) are
+// scanned with the reference's operations instead (24,000 such positions x 8,192 codes 1,048 us,
+// others 44.5; finding the largest component costs 0.7 us of 34 for 500 positions).
 // 409,600 positions x 8,192 codes, fp32: 1292 -> 453 us, 7.4e12 pairs per second; bound by the
 // sum of the two (about 180 VALU and 128 MFMA cycles per 1,024 pairs: the fp32 MFMAs measured
 // without overlap).
@@ -136,7 +159,7 @@ __device__ __forceinline__ void exact_search(const T* __restrict__ z, const T* _
                                              const T* __restrict__ codebook, const T* __restrict__ cb_norm, int64_t P,
                                              int E, int32_t* __restrict__ indices, T* __restrict__ quantized,
                                              float4* cb /* components 0, 2, 1, 3: lane half h reads (h, 2 + h) */,
-                                             T* cbn, float* s_best, int* s_chunk) {
+                                             T* cbn, unsigned* s_em, float* s_best, int* s_chunk) {
   static_assert(SPLIT == 1 || (SPLIT == 4 && PG == 1), "whole scans, or quarters of one column group");
   constexpr bool HALF = sizeof(T) == 2;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -163,15 +186,26 @@ __device__ __forceinline__ void exact_search(const T* __restrict__ z, const T* _
 #pragma unroll
   for (int g = 0; g < PG; g++) { best[g] = INFINITY; chunk[g] = 0x7fffffff; }
   const f32x16 zero = {};
+  unsigned em = 0;   // FP32: largest |component| of the staged codes, as bits (a code with a non-finite one has no finite dot)
   for (int base = 0; base < E; base += VQ_STAGE) {
     const int n = min(VQ_STAGE, E - base), nr = (n + VQ_CHUNK - 1) / VQ_CHUNK * VQ_CHUNK;
     __syncthreads();   // the previous stage is no longer read
     // Past the last code: zeros at an infinite norm.
     for (int i = threadIdx.x; i < nr; i += VQ_THREADS) {
       const T* e = codebook + (int64_t)(base + (i < n ? i : 0)) * 4;
-      cb[i] = i < n ? make_float4((float)e[0], (float)e[2], (float)e[1], (float)e[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float4 v = i < n ? make_float4((float)e[0], (float)e[2], (float)e[1], (float)e[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+      cb[i] = v;
+      if constexpr (!HALF) {
+        const unsigned m = max4_bits(v);
+        em = m < 0x7f800000u ? max(em, m) : em;
+      }
       cbn[i] = i < n ? cb_norm[base + i] : (T)INFINITY;
     }
+    if constexpr (!HALF && SPLIT == 4)
+      if (base + VQ_STAGE >= E) {
+        em = wave_max(em);
+        if (lane == 0) s_em[wave] = em;
+      }
     __syncthreads();
     for (int c0 = SPLIT == 1 ? 0 : wave * VQ_CHUNK; c0 < nr; c0 += SPLIT * VQ_CHUNK) {
       float m[PG][2];
@@ -232,6 +266,15 @@ __device__ __forceinline__ void exact_search(const T* __restrict__ z, const T* _
       }
     }
   }
+  if constexpr (!HALF) {   // em over the workgroup
+    if constexpr (SPLIT == 1) {
+      __syncthreads();   // the last stage, whose memory s_em shares, is no longer read
+      em = wave_max(em);
+      if (lane == 0) s_em[wave] = em;
+      __syncthreads();
+    }
+    em = max(max(s_em[0], s_em[1]), max(s_em[2], s_em[3]));
+  }
   // The two lane halves (codes 0-3 and 4-7 of every eight), then the four waves.
 #pragma unroll
   for (int g = 0; g < PG; g++) {
@@ -273,8 +316,12 @@ __device__ __forceinline__ void exact_search(const T* __restrict__ z, const T* _
     T zt[4];
 #pragma unroll
     for (int c = 0; c < 4; c++) zt[c] = z[pos * 4 + c];
+    if constexpr (!HALF) {   // a double may overflow: the plain scan
+      const unsigned zm = max4_bits(make_float4(zt[0], zt[1], zt[2], zt[3]));
+      if (zm < 0x7f800000u && __uint_as_float(zm) * __uint_as_float(em) >= 0x1p124f) found = 0x7fffffff;
+    }
     if (found >= E) {
-      // No real code has the distance (a norm of -inf beside the padding's +inf): the plain scan.
+      // (Also where no real code has the distance: a norm of -inf beside the padding's +inf.)
       const float zs[4] = {(float)zt[0], (float)zt[1], (float)zt[2], (float)zt[3]};
       T d0 = (T)0.f;
       for (int code = 0; code < E; code++) {
@@ -301,7 +348,8 @@ __global__ __launch_bounds__(VQ_THREADS, SPLIT == 1 ? 4 : 3) void vq_nearest4_ke
   __shared__ __attribute__((aligned(16))) T cbn[VQ_STAGE];
   __shared__ float s_best[SPLIT == 4 ? 128 : 1];
   __shared__ int s_chunk[SPLIT == 4 ? 128 : 1];
-  exact_search<T, PG, SPLIT>(z, z_norm, codebook, cb_norm, P, E, indices, quantized, cb, cbn, s_best, s_chunk);
+  __shared__ unsigned s_em[4];
+  exact_search<T, PG, SPLIT>(z, z_norm, codebook, cb_norm, P, E, indices, quantized, cb, cbn, s_em, s_best, s_chunk);
 }
 
 // 2^e of a nonzero value from its absolute bits; `zero` for 0. Whether it may be scaled.
@@ -346,12 +394,11 @@ __global__ __launch_bounds__(VQ_THREADS, 4) void vq_nearest4_bounds_kernel(
   const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
   auto load4 = [](const float* v) { return make_float4(v[0], v[1], v[2], v[3]); };
   auto abs_bits = [](float v) { return (unsigned)__float_as_int(v) & 0x7fffffffu; };
-  auto max4 = [&](float4 v) { return max(max(abs_bits(v.x), abs_bits(v.y)), max(abs_bits(v.z), abs_bits(v.w))); };
   // Largest component and squared norm of the codebook, as absolute bits (a NaN is the largest).
   unsigned em = 0, nm = 0;
 #pragma unroll 8
   for (int i = threadIdx.x; i < E; i += VQ_THREADS) {
-    em = max(em, max4(load4(codebook + (int64_t)i * 4)));
+    em = max(em, max4_bits(load4(codebook + (int64_t)i * 4)));
     nm = max(nm, abs_bits(cb_norm[i]));
   }
 #pragma unroll
@@ -375,14 +422,14 @@ __global__ __launch_bounds__(VQ_THREADS, 4) void vq_nearest4_bounds_kernel(
       const float v[4] = {zv.x, zv.y, zv.z, zv.w};
       zn = z_norm ? z_norm[pos] : squared_norm4<float>(v);
     }
-    const unsigned zm = max4(zv);
+    const unsigned zm = max4_bits(zv);
     f16x8 zb[2];
 #pragma unroll
     for (int g = 0; g < 2; g++) {
       const int64_t q = p0 + 32 * g + col;
       const float4 v4 = q < P ? load4(z + q * 4) : zero4;
       const float v[4] = {v4.x, v4.y, v4.z, v4.w};
-      const unsigned m = max4(v4);
+      const unsigned m = max4_bits(v4);
       const int zs = bits_scalable(m) ? 10 - bits_exponent(m, 10) : 0;
       const int bs = min(max(zs + es - ns, -14), 15);
 #pragma unroll
@@ -512,7 +559,8 @@ __global__ __launch_bounds__(VQ_THREADS, 4) void vq_nearest4_bounds_kernel(
   if (exact) {
     __syncthreads();
     exact_search<float, 2, 1>(z, z_norm, codebook, cb_norm, P, E, indices, quantized, reinterpret_cast<float4*>(lds),
-                              reinterpret_cast<float*>(lds + VQ_STAGE * 16), nullptr, nullptr);
+                              reinterpret_cast<float*>(lds + VQ_STAGE * 16), reinterpret_cast<unsigned*>(lds), nullptr,
+                              nullptr);
   }
 }
 

@@ -175,3 +175,28 @@ def test_search_from_bounds(pkg, dev, kind, positions, entries) -> None:
     with np.errstate(invalid="ignore", over="ignore"):
         want, _ = ovq.quantize4(flat[rows], cb, np.float32)
     np.testing.assert_array_equal(idx[rows], want)
+
+
+@pytest.mark.parametrize("kind", ["doubled dot overflows", "around overflow", "subnormal", "around underflow"])
+@pytest.mark.parametrize("positions", [70, 24700])
+def test_search_beyond_the_normal_range(pkg, dev, kind, positions) -> None:
+    """FP32 distances that overflow or are subnormal, below 24,577 positions and above: a dot whose
+    double overflows beside an infinite sum of norms is a NaN, which wins. Every row equals the
+    oracle's."""
+    rng = np.random.default_rng(positions)
+    cb, flat = rng.normal(size=(130, 4)), rng.normal(size=(positions, 4))
+    if kind == "doubled dot overflows":
+        cb, flat = cb * 0, flat * 1e19
+        cb[100] = 1.2e19, 1.2e19, 0, 0
+        cb[77] = 1.1e19, 0, 0, 0
+        flat[:2] = [1e19, 1e19, 0, 0], [1.6e19, 0, 0, 0]
+    else:
+        lo, hi = {"around overflow": (55, 66), "subnormal": (-76, -70), "around underflow": (-68, -55)}[kind]
+        cb, flat = (v * np.exp2(rng.integers(lo, hi, (len(v), 1))) for v in (cb, flat))
+    cb, flat = cb.astype(np.float32), flat.astype(np.float32)
+    idx, _, _ = _search(pkg, dev, flat, cb, torch.float32)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want, _ = ovq.quantize4(flat, cb, np.float32)
+    if kind == "doubled dot overflows":
+        assert want[0] == 100 and want[1] == 77
+    np.testing.assert_array_equal(idx, want)
