@@ -106,11 +106,14 @@ __device__ __forceinline__ float src_x(const SrcConvParams& p, const SrcTap& tp,
 // MASKED (kernels of at most 32 taps, tensors within 31 bits of bytes): a position's valid taps
 // are a 32-bit mask made once, and a load is a buffer load at the window start plus a scalar
 // (channel, tap) offset, sent out of range where the mask has no bit: four VALU
-// operations per im2col value against twelve with bounds checks. The fp32 MFMAs do not
+// operations per im2col value against twelve with bounds checks. The scalar offset stays
+// within the buffer's length, so that what is left of it after the offset does not wrap and the
+// position sent out of range is (a step's k past the last, or a tap that lies in the padding
+// for every position, has an offset beyond it). The fp32 MFMAs do not
 // overlap the VALU, so the gather is on the critical path.
 //
 // 64 -> 64 at 32 x 40 x 40: 375 us on the VALU, 235 with the index arithmetic on the scalar
-// unit, 155 now (73 TFLOP/s; the MFMAs alone are 79 us, 100 with 800 workgroups on 256 CUs).
+// unit, 155 now (73 TFLOP/s; at 2.2 GHz the MFMAs alone are 79 us, 100 with 800 workgroups on 256 CUs).
 template <bool MASKED>
 __global__ __launch_bounds__(SC_THREADS, 4) void src_conv_kernel(SrcConvParams p) {
   touch_args(p);
@@ -164,8 +167,9 @@ __global__ __launch_bounds__(SC_THREADS, 4) void src_conv_kernel(SrcConvParams p
       const int k = base + lane;
       const int c = udiv(k, p.dv_taps), tap = k - c * p.taps;
       const int kd = udiv(tap, p.dv_khw), r = tap - kd * p.khw, kh = udiv(r, p.dv_kw), kw = r - kh * p.KW;
-      koff = ((unsigned)c * (unsigned)p.xsC + (unsigned)((kd * p.H + kh) * p.W + kw) * (unsigned)p.xsV) * 2u;
+      const unsigned o = ((unsigned)c * (unsigned)p.xsC + (unsigned)((kd * p.H + kh) * p.W + kw) * (unsigned)p.xsV) * 2u;
       kbit = k < p.complete ? 1u << tap : 0u;
+      koff = kbit ? min(o, p.records) : 0u;
     }
 #pragma unroll
     for (int i = 0; i < NX; i++) {

@@ -66,6 +66,23 @@ def test_source_conv_tiles_and_tails(pkg, dev, case) -> None:
         np.testing.assert_array_equal(_bits(got)[~nan], _bits(want)[~nan])
 
 
+@pytest.mark.parametrize(("grid", "channels", "kernel", "padding"), [
+    ((6, 7, 9), 32, (3, 3, 3), 1),   # the last step's k past the last channel, two bytes beyond the tensor
+    ((6, 7, 9), 96, (3, 3, 3), 1),
+    ((1, 3, 7), 4, (5, 1, 1), 2),    # taps of the last channel that lie in the padding everywhere, ten bytes beyond
+    ((1, 3, 5), 3, (5, 1, 1), 2),
+    ((3, 1, 2), 33, (2, 3, 5), 3),
+], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_source_conv_gather_offsets_past_the_tensor(pkg, dev, grid, channels, kernel, padding) -> None:
+    """One NCDHW batch item, whose last step has (channel, tap) offsets just past the tensor's end:
+    those lanes read zeros."""
+    rng = np.random.default_rng(channels)
+    x = rng.normal(size=(1, channels, *grid)).astype(np.float16)
+    w = rng.normal(size=(35, channels, *kernel)).astype(np.float16)
+    y = pkg.ops.conv3d_half(_dev(x, dev), _dev(w, dev), None, padding=padding, stride=1)
+    np.testing.assert_array_equal(_bits(y.cpu().numpy()), _bits(so.conv3d_half(x, w, None, padding=padding, stride=1)))
+
+
 def test_source_conv_channels_last_gives_the_same_bits(pkg, dev) -> None:
     x, w, b = conv_case(95, 35, (3, 3, 3), True)
     xd = _dev(x, dev)
