@@ -1041,12 +1041,10 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 3) void attention_tile_kernel(At
   if (nst > 1) issue(1);
   for (int st = 0; st < nst; st++) {
     // This wave's share of stage st has landed when at most stage st + 1's is outstanding; after
-    // the barrier so have the others', and stage st - 1's slot is free.
+    // the barrier so have the others', and stage st - 1's slot is read.
     if (st + 1 < nst) vmcnt_wait<DK>();
     else vmcnt_wait<0>();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    ring_barrier();
     if (st + 2 < nst) issue(st + 2);
     const E* sb = smem + (st % 3) * 2 * SUB;
     const unsigned slot = (unsigned)((st % 3) * 2 * SUB) * 2u;

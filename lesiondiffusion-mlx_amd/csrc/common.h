@@ -315,4 +315,15 @@ __device__ __forceinline__ void vmcnt_wait() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
+// Workgroup barrier after which a slot of an LDS ring is given to a DMA: every wave's reads of it
+// have returned. (The consumers of a read may be scheduled past the barrier, and with them the wait
+// that the compiler places; a DMA is not ordered behind another wave's reads.) Unlike
+// __syncthreads, outstanding DMAs of other slots are not awaited.
+__device__ __forceinline__ void ring_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 }  // namespace ldx

@@ -649,12 +649,10 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void attention_planes_kernel(
   if (nb > 1) dma(1);
   for (int it = 0; it < nb; it++) {
     // This wave's share of block it has landed when at most block it + 1's DMAs are outstanding;
-    // after the barrier so have the others', and the slot of block it - 1 is free.
+    // after the barrier so have the others', and the slot of block it - 1 is read.
     if (it + 1 < nb) vmcnt_wait<NF>();
     else vmcnt_wait<0>();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    ring_barrier();
     if (it + 2 < nb) dma(it + 2);
     const int slot = it % RING;
     f32x16 sh = {}, sx = {};

@@ -260,3 +260,14 @@ def test_voxel_pitch_and_head_views(pkg, shape) -> None:
         assert pkg.ops._interleaved(t, "q", 8) == (view.data_ptr(), view.stride()[:3])
     with pytest.raises(ValueError, match="head_dim must be contiguous"):
         pkg.ops._interleaved(torch.empty(1, 24, 7).transpose(1, 2), "q", 8)
+
+
+def test_bare_barriers_wait_for_lds_reads() -> None:
+    """A bare s_barrier does not wait for a wave's LDS reads, so handing a ring slot to a DMA after
+    one races them: only ``ring_barrier`` (common.h), which waits first, uses it."""
+    csrc = REPO / "lesiondiffusion-mlx_amd" / "csrc"
+    uses = [(f.name, line.strip()) for f in sorted(csrc.iterdir()) for line in f.read_text().splitlines()
+            if "amdgcn_s_barrier" in line]
+    assert uses == [("common.h", "__builtin_amdgcn_s_barrier();")]
+    body = (csrc / "common.h").read_text().split("void ring_barrier() {")[1].split("}")[0]
+    assert body.index("s_waitcnt(0xC07F)") < body.index("s_barrier")
