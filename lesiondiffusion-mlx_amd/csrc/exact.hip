@@ -541,12 +541,12 @@ __global__ __launch_bounds__(256) void attention_split_kernel(SplitAttnParams p)
 //
 // Softmax: the base moves only when a lane's 16 probabilities sum to 128 (a score about 7 above
 // it), seen on the sum that is needed anyway, so that no maximum is taken and the accumulators
-// are rarely rescaled; the block's probabilities are then made again. Probabilities are kept as p 2^8 (scaled after exp2: in its argument the 8 would cost
-// three of its bits, 2.0e-7 -> 2.9e-7 against float64): hi = half(p), lo = half(p - hi) unscaled,
-// one v_cvt and one mixed fused multiply-add; what lo loses to fp16's subnormal step is below
-// 2^-32 of the largest probability. Ph Vh, Pl Vh and 2^11 Ph Vl have an accumulator each.
+// are rarely rescaled; the block's probabilities are then made again. Probabilities are split as
+// in the kernel above, hi = half(p), lo = half((p - hi) 2^11), by packed conversions (an unscaled lo
+// is subnormal for small probabilities: 2.3e-5 of a sum of many at 2^-18, 3e-6 scaled).
+// Ph Vh has one accumulator, 2^11 (Pl Vh + Ph Vl) the other.
 // Per 32 x 32 block 12 (D = 32) MFMAs and about 110 VALU operations, 16 of them exp2; VALU-bound.
-// 23,104 tokens, two 32-wide heads: 1250 -> 479 us (285 TFLOP/s of FP32 products).
+// 23,104 tokens, two 32-wide heads: 1248 -> 481 us (284 TFLOP/s of FP32 products).
 struct PlanesAttnParams {
   int B, H, L, LK, nblk, S, per;   // key blocks of 32, key ranges, blocks per range
   const float* q; int64_t qs0, qs1, qs2;
@@ -639,11 +639,11 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void attention_planes_kernel(
   };
   auto frag = [&](int slot, int f) { return *reinterpret_cast<const f16x8*>(smem + slot * BLK + f * 512 + lane * 8); };
 
-  f32x16 oh[DB], ol[DB], ox[DB];
+  f32x16 oh[DB], ox[DB];
 #pragma unroll
   for (int i = 0; i < DB; i++)
 #pragma unroll
-    for (int e = 0; e < 16; e++) oh[i][e] = ol[i][e] = ox[i][e] = 0.f;
+    for (int e = 0; e < 16; e++) oh[i][e] = ox[i][e] = 0.f;
   float mb = -1e30f, l = 0.f;
   dma(0);
   if (nb > 1) dma(1);
@@ -686,14 +686,14 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void attention_planes_kernel(
       float q[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int e = 0; e < 16; e++) {
-        t[e] = __builtin_amdgcn_exp2f(t[e]) * 256.0f;
+        t[e] = __builtin_amdgcn_exp2f(t[e]);
         q[e & 3] += t[e];
       }
       sum = (q[0] + q[1]) + (q[2] + q[3]);
     };
     relative();
     probabilities();
-    if (__ballot(sum > 32768.f)) {   // a score above the base by up to 7 (the first block's: by 1e30)
+    if (__ballot(sum > 128.f)) {   // a score above the base by up to 7 (the first block's: by 1e30)
       const float old = mb;
       mb = 0.f;
       relative();   // the scores themselves
@@ -703,18 +703,22 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void attention_planes_kernel(
 #pragma unroll
       for (int db = 0; db < DB; db++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) { oh[db][e] *= alpha; ol[db][e] *= alpha; ox[db][e] *= alpha; }
+        for (int e = 0; e < 16; e++) { oh[db][e] *= alpha; ox[db][e] *= alpha; }
       relative();
       probabilities();
     }
     l += sum;
     f16x8 ph[2], pl[2];
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
-      asm volatile("" : "+v"(t[e]));   // one fp32 value feeds both halves
-      const f16 hi = (f16)t[e];
-      ph[e >> 3][e & 7] = hi;
-      pl[e >> 3][e & 7] = (f16)(t[e] - (float)hi);
+    for (int e = 0; e < 16; e += 2) {
+      asm volatile("" : "+v"(t[e]), "+v"(t[e + 1]));   // one fp32 value feeds both halves
+      f16x2 hi = {(f16)t[e], (f16)t[e + 1]};
+      asm volatile("" : "+v"(hi));   // one packed conversion
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        ph[e >> 3][(e & 7) + i] = hi[i];
+        pl[e >> 3][(e & 7) + i] = (f16)__builtin_fmaf(t[e + i] - (float)hi[i], 2048.0f, 0.0f);   // v_fma_mixlo / hi
+      }
     }
 #pragma unroll
     for (int ks = 0; ks < 2; ks++)
@@ -722,7 +726,7 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void attention_planes_kernel(
       for (int db = 0; db < DB; db++) {
         const f16x8 vh = frag(slot, 2 * NF + ks * DB + db), vl = frag(slot, 3 * NF + ks * DB + db);
         oh[db] = mfma_h(vh, ph[ks], oh[db]);
-        ol[db] = mfma_h(vh, pl[ks], ol[db]);
+        ox[db] = mfma_h(vh, pl[ks], ox[db]);
         ox[db] = mfma_h(vl, ph[ks], ox[db]);
       }
   }
@@ -736,7 +740,7 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void attention_planes_kernel(
       for (int j = 0; j < 4; j++) {
         f32x4 out;
 #pragma unroll
-        for (int r = 0; r < 4; r++) out[r] = oh[db][4 * j + r] + (ol[db][4 * j + r] + ox[db][4 * j + r] * (1.0f / 2048.0f));
+        for (int r = 0; r < 4; r++) out[r] = oh[db][4 * j + r] + ox[db][4 * j + r] * (1.0f / 2048.0f);
         dst[(db * 8 + 2 * j + hf) * 32 + col] = out;
       }
     if (hf == 0) dst[D / 4 * 32 + col] = (f32x4){mb, l, 0.f, 0.f};
@@ -750,7 +754,7 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void attention_planes_kernel(
         f32x4 out;
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          out[r] = (oh[db][4 * j + r] + (ol[db][4 * j + r] + ox[db][4 * j + r] * (1.0f / 2048.0f))) * inv;
+          out[r] = (oh[db][4 * j + r] + ox[db][4 * j + r] * (1.0f / 2048.0f)) * inv;
         *reinterpret_cast<f32x4*>(orow + db * 32 + j * 8 + 4 * hf) = out;
       }
   }

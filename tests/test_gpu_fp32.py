@@ -344,6 +344,25 @@ def test_fp32_attention_key_ranges(pkg, dev, d, batch, heads, lq, lk) -> None:
 
 
 @pytest.mark.parametrize("d", [32, 64])
+def test_fp32_attention_of_many_small_probabilities(pkg, dev, d) -> None:
+    """Every 64th key's score is 11 to 18 (log2 units) above those of the others, which are equal and
+    alone have values: the output is the sum of their small probabilities, in which equal rounding
+    errors add. Bound: a probability keeps 2^-22 of itself (hi / lo), the rounding of its exponent
+    (2^-23 of 18) and exp2 2^-20.4, the sums of 47 blocks 2^-19 in the worst order: 4e-6 of the value."""
+    lk, lq = 1504, 256
+    gaps = np.linspace(11, 18, lq)
+    q = np.zeros((1, lq, d), np.float32)
+    q[..., 0] = gaps / 1.44269504088896341
+    k, v = np.zeros((1, lk, d), np.float32), np.ones((1, lk, d), np.float32)
+    k[0, 5::64, 0], v[0, 5::64] = 1, 0
+    high = len(range(5, lk, 64))
+    got = host(pkg.ops.flash_attention(dev32(q, dev), dev32(k, dev), dev32(v, dev), heads=1, scale=1.0))
+    p = np.exp2(-q[0, :, 0].astype(np.float64) * np.log2(np.e))
+    want = ((lk - high) * p / (high + (lk - high) * p))[None, :, None]
+    np.testing.assert_allclose(got, np.broadcast_to(want, got.shape), rtol=4e-6, atol=0)
+
+
+@pytest.mark.parametrize("d", [32, 64])
 def test_fp32_attention_split_kernel_agrees_with_the_valu_kernel(pkg, dev, monkeypatch, d) -> None:
     """The split-fp16 MFMA kernel and the FP32 VALU flash kernel (LDX_ATTN_F32=valu) on the
     same ragged inputs: both within FP32 error of each other."""
