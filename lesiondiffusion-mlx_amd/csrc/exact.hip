@@ -60,21 +60,21 @@ __global__ void pack_weight_exact_kernel(const float* __restrict__ w, int O, int
   }
 }
 
-// v / (1 + exp(-v)) in fp32, within an ulp or two: exp(-v) = 2^n 2^f with n the nearest integer
-// to -v log2(e) and f the rest from log2(e) in two parts, and the quotient from the hardware
-// reciprocal with a Newton step, one residual correction and v_div_fixup (-0 for large
-// negative v, NaN for -inf, as the division gives). About 20 issue slots against about 45 of
-// expf and the compiler's division.
+// v / (1 + exp(-v)) in fp32, within an ulp or two down to where exp(-v) overflows: exp(-v) = 2^n 2^f
+// with n the nearest integer to -v log2(e) and f the rest from log2(e) in two parts, and the quotient
+// from the hardware reciprocal (1 ulp) with one residual correction and v_div_fixup (-0 for large
+// negative v, NaN for -inf, as the division gives). Numerator and denominator are quartered: the
+// reciprocal of a denominator above 2^126 would be subnormal, which v_rcp_f32 flushes. About 20 issue
+// slots against about 45 of expf and the compiler's division.
 __device__ __forceinline__ float silu32(float v) {
   const float a = __builtin_amdgcn_fmed3f(v, -256.f, 256.f);
   const float n = __builtin_rintf(a * -1.44269504f);
   const float f = __builtin_fmaf(a, -1.92596299e-8f, __builtin_fmaf(a, -1.44269502f, -n));
-  const float d = 1.0f + __builtin_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
-  float r = __builtin_amdgcn_rcpf(d);
-  r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
-  float q = v * r;
-  q = __builtin_fmaf(__builtin_fmaf(-q, d, v), r, q);
-  return __builtin_amdgcn_div_fixupf(q, d, v);
+  const float d = 0.25f + __builtin_ldexpf(__builtin_amdgcn_exp2f(f), (int)n - 2), u = v * 0.25f;
+  const float r = __builtin_amdgcn_rcpf(d);
+  float q = u * r;
+  q = __builtin_fmaf(__builtin_fmaf(-q, d, u), r, q);
+  return __builtin_amdgcn_div_fixupf(q, d, u);
 }
 __device__ __forceinline__ float gelu_erf32(float v) { return v * (1.0f + erff(v * 0.70710678118654752f)) * 0.5f; }
 

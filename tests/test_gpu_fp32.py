@@ -188,6 +188,26 @@ def test_fp32_silu_of_extreme_values(pkg, dev) -> None:
     np.testing.assert_allclose(host(y)[0, 0, 0, 0], want, rtol=4 * 2.0 ** -22, atol=2.0 ** -35)
 
 
+def test_fp32_silu_over_its_range(pkg, dev) -> None:
+    """silu as the epilogue of a 1x1x1 identity conv, whose sums are the inputs themselves (at most 22
+    significant bits), within 3 ulps (exp2 and the quotient one each, the exponent's rest a half) down to
+    where 1 + exp(-v) overflows, and within the least normal value's 2^5 beyond; -inf gives NaN."""
+    rng = np.random.default_rng(4)
+    v = np.concatenate([np.linspace(-88.7, 88, 60000), np.linspace(-88.72, -87, 4000), rng.normal(size=4000) * 8,
+                        -np.exp2(rng.uniform(-60, 6, 2000)), np.exp2(rng.uniform(-60, 15, 2000)),
+                        [0.0, -88.72, -88.0, -87.4, -89.0, -104.0, -300.0, 6e4]])
+    v = v[:len(v) // 32 * 32].astype(np.float32)
+    v = (v.view(np.uint32) & ~np.uint32(3)).view(np.float32)   # 22 bits
+    x = torch.from_numpy(v.reshape(1, 1, 1, -1, 32)).to(dev)
+    y = pkg.ops.nax_conv3d(x, pkg.ops.pack_weight(torch.eye(32, device=dev)), act="silu")
+    sums = host(pkg.ops.nax_conv3d(x, pkg.ops.pack_weight(torch.eye(32, device=dev)))).ravel()
+    want = sums / (1 + np.exp(-sums))
+    got = host(y).ravel()
+    far = sums < -88.72
+    np.testing.assert_allclose(got[~far], want[~far], rtol=3 * 2.0 ** -23, atol=0)
+    np.testing.assert_allclose(got[far], want[far], rtol=0, atol=2.0 ** -121)
+
+
 @pytest.mark.parametrize("k", [1, 3])
 def test_fp32_unaligned_concat_with_batched_affine(pkg, dev, k) -> None:
     """Channel counts that are not multiples of 4 (element-wise input reads), two batch items
