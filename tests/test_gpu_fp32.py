@@ -288,6 +288,17 @@ def test_fp32_group_norm_of_large_tensors(pkg, dev, shape, c1, groups, mean) -> 
     np.testing.assert_allclose(aff, want, rtol=2e-6, atol=2e-6 + 2.0 ** -20 * abs(mean))
 
 
+@pytest.mark.parametrize("batch", [2, 5])
+def test_fp32_group_norm_of_an_item_does_not_depend_on_its_batch(pkg, dev, batch) -> None:
+    """Each item's statistics in the two-launch form: the bits of that item alone."""
+    rng = np.random.default_rng(batch)
+    x = dev32(rng.normal(size=(batch, 64, 66, 67, 16)), dev)
+    gamma, beta = (dev32(rng.normal(size=16), dev) for _ in range(2))
+    aff = pkg.ops.group_norm_affine(x, gamma, beta, groups=8, eps=1e-5)
+    for b in range(batch):
+        assert torch.equal(aff[b:b + 1], pkg.ops.group_norm_affine(x[b:b + 1], gamma, beta, groups=8, eps=1e-5))
+
+
 @pytest.mark.parametrize(("lq", "lk", "d"), [(64, 3, 16), (300, 300, 32), (129, 77, 64), (8, 8, 16)])
 def test_fp32_attention_matches_float64(pkg, dev, lq, lk, d) -> None:
     rng = np.random.default_rng(lq + lk + d)
