@@ -28,9 +28,9 @@ void set_error(const char* fmt, ...);
 int fail(const char* fmt, ...);  // set_error + return LDX_EINVAL
 int check_launch(const char* what);  // hipGetLastError -> LDX_EHIP / LDX_OK
 
-// Merges per-chunk GroupNorm partials [batch][nchunks][groups][3] into (scale, offset).
-int launch_gn_finalize(const float* partial, int nchunks, int batch, int C, int groups, const float* gamma,
-                       const float* beta, float eps, float* affine, hipStream_t st);
+// Merges per-chunk GroupNorm partials [batch][nchunks][groups][3] of an FP32 tensor into (scale, offset).
+int launch_gn_finalize_f32(const float* partial, int nchunks, int batch, int C, int groups, const float* gamma,
+                           const float* beta, float eps, float* affine, hipStream_t st);
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 

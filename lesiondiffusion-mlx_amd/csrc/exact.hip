@@ -117,7 +117,9 @@ __global__ __launch_bounds__(256) void gn_f32_kernel(const float* __restrict__ x
 // so the reads are whole contiguous rows, and gn_finalize_kernel merges the chunks. A thread
 // owns V channels (16 bytes) of every vpi-th voxel, eight voxels' loads in flight: their mean,
 // then their squared deviations from it, merged into the running moments (Chan), one division
-// per eight voxels; no shift, no cancellation, and the order is fixed. Memory-bound; both
+// per eight voxels; no shift, no cancellation, and the order is fixed. A mean is never squared (of
+// the first values d is the mean itself, and merge() with an empty set squares it): values of any
+// size have statistics where their deviations' squares do not overflow. Memory-bound; both
 // launches: 76 x 128 x 152 x 16 (95 MB) 2752 -> 22 us (4.3 TB/s), 128 x 160 x 160 x 96
 // (1.26 GB) 44.6 ms -> 215 us (5.9 TB/s), 19 x 32 x 38 x 64 89 -> 8.0 us.
 template <int V>
@@ -141,21 +143,23 @@ __global__ __launch_bounds__(256) void gn_f32_partial_kernel(const float* __rest
       vec h[8];
 #pragma unroll
       for (int u = 0; u < 8; u++) h[u] = at(v + u * vpi);
-      const vec bm = (((h[0] + h[1]) + (h[2] + h[3])) + ((h[4] + h[5]) + (h[6] + h[7]))) * 0.125f;
+      vec bm = (vec)(0.f);
+#pragma unroll
+      for (int u = 0; u < 8; u += 2) bm += h[u] * 0.125f + h[u + 1] * 0.125f;   // (their sum may overflow)
       vec q = (vec)(0.f);
 #pragma unroll
       for (int u = 0; u < 8; u++) q += (h[u] - bm) * (h[u] - bm);
       const float f = 8.f / (n + 8.f);
       const vec d = bm - mean;
       mean += d * f;
-      m2 += q + d * d * (n * f);
+      m2 += q + d * (d * (n * f));
       n += 8.f;
     }
     for (; v < v_end; v += vpi) {
       const vec d = at(v) - mean;
       n += 1.f;
       mean += d * (1.f / n);
-      m2 += d * d * ((n - 1.f) / n);
+      m2 += d * (d * ((n - 1.f) / n));
     }
   }
   // The voxel slots' moments of a channel, folded in halves.
@@ -168,7 +172,7 @@ __global__ __launch_bounds__(256) void gn_f32_partial_kernel(const float* __rest
   for (int k = vpi; k > 1;) {
     const int half = (k + 1) / 2;
     __syncthreads();
-    if (active && sub + half < k) {
+    if (active && sub + half < k && s_n[sub + half] > 0.f) {   // (slots fill from the first)
       const int o = sub + half;
       const float on = s_n[o];
       Moments m = {n, 0.f, 0.f};
@@ -185,8 +189,8 @@ __global__ __launch_bounds__(256) void gn_f32_partial_kernel(const float* __rest
   __syncthreads();
   const int gs = C / G;
   for (int g = t; g < G; g += 256) {
-    Moments m = {0.f, 0.f, 0.f};
-    for (int c = g * gs; c < (g + 1) * gs; c++) m = merge(m, Moments{s_n[0], s_mean[c], s_m2[c]});
+    Moments m = {s_n[0], s_mean[g * gs], s_m2[g * gs]};
+    for (int c = g * gs + 1; c < (g + 1) * gs; c++) m = merge(m, Moments{s_n[0], s_mean[c], s_m2[c]});
     float* out = partial + (((int64_t)b * gridDim.x + blockIdx.x) * G + g) * 3;
     out[0] = m.n; out[1] = m.mean; out[2] = m.m2;
   }
@@ -1689,7 +1693,7 @@ extern "C" int ldx_group_norm_affine_f32_ws(const float* x0, int64_t x0_pitch, i
       hipLaunchKernelGGL(gn_f32_partial_kernel<1>, grid, dim3(256), 0, st, x0, x0_pitch, c0, xb, pb, C, groups, voxels,
                          chunk, part);
     if (int rc = check_launch("group_norm_affine_f32: partial")) return rc;
-    return launch_gn_finalize(part, (int)nchunks, batch, C, groups, gamma, beta, eps, affine, st);
+    return launch_gn_finalize_f32(part, (int)nchunks, batch, C, groups, gamma, beta, eps, affine, st);
   }
   hipLaunchKernelGGL(gn_f32_kernel, dim3(groups, batch), dim3(256), 0, st, x0, x0_pitch, c0, xb, pb, C, groups, voxels,
                      gamma, beta, eps, affine);

@@ -212,19 +212,23 @@ __global__ __launch_bounds__(256) void gn_partial_kernel(
 }
 
 // Pass 2: one workgroup per (group, batch item) merges the chunk partials in a
-// fixed tree order and writes the (scale, offset) pairs of the group's channels.
+// fixed tree order and writes the (scale, offset) pairs of the group's channels. SHIFT (FP32
+// tensors): means relative to the first chunk's, whose squares may overflow where the
+// deviations' do not (merging into an empty set squares a mean).
+template <bool SHIFT>
 __global__ __launch_bounds__(256) void gn_finalize_kernel(
     const float* __restrict__ partial, int nchunks, int C, int G, const float* __restrict__ gamma,
     const float* __restrict__ beta, float eps, float* __restrict__ affine) {
   __shared__ float red[12];
   const int g = blockIdx.x, b = blockIdx.y, t = threadIdx.x;
+  const float shift = SHIFT ? partial[((int64_t)b * nchunks * G + g) * 3 + 1] : 0.f;
   Moments m = {0.f, 0.f, 0.f};
   for (int j = t; j < nchunks; j += 256) {
     const float* pp = partial + (((int64_t)b * nchunks + j) * G + g) * 3;
-    m = merge(m, Moments{pp[0], pp[1], pp[2]});
+    m = merge(m, Moments{pp[0], SHIFT ? pp[1] - shift : pp[1], pp[2]});
   }
   const Moments tot = block_merge256(m, red);
-  const float mean = tot.mean;
+  const float mean = SHIFT ? shift + tot.mean : tot.mean;
   const float var = tot.n > 0.f ? tot.m2 / tot.n : 0.f;
   const float rstd = 1.0f / sqrtf(var + eps);
   const int gs = C / G;
@@ -235,11 +239,11 @@ __global__ __launch_bounds__(256) void gn_finalize_kernel(
   }
 }
 
-int launch_gn_finalize(const float* partial, int nchunks, int batch, int C, int groups, const float* gamma,
-                       const float* beta, float eps, float* affine, hipStream_t st) {
-  hipLaunchKernelGGL(gn_finalize_kernel, dim3(groups, batch), dim3(256), 0, st, partial, nchunks, C, groups, gamma,
-                     beta, eps, affine);
-  return check_launch("group_norm_affine: finalize");
+int launch_gn_finalize_f32(const float* partial, int nchunks, int batch, int C, int groups, const float* gamma,
+                           const float* beta, float eps, float* affine, hipStream_t st) {
+  hipLaunchKernelGGL(gn_finalize_kernel<true>, dim3(groups, batch), dim3(256), 0, st, partial, nchunks, C, groups,
+                     gamma, beta, eps, affine);
+  return check_launch("group_norm_affine_f32: finalize");
 }
 
 // Small tensors (coarse UNet levels): one launch, one workgroup per (group, batch item).
@@ -633,7 +637,9 @@ static int group_norm_affine_impl(const void* x0, int64_t p0, int32_t c0, const 
                        (int)nchunks);
   int rc = check_launch("group_norm_affine: partial");
   if (rc) return rc;
-  return launch_gn_finalize(part, (int)nchunks, batch, C, groups, gamma, beta, eps, affine, st);
+  hipLaunchKernelGGL(gn_finalize_kernel<false>, dim3(groups, batch), dim3(256), 0, st, part, (int)nchunks, C, groups,
+                     gamma, beta, eps, affine);
+  return check_launch("group_norm_affine: finalize");
 }
 
 extern "C" int ldx_group_norm_affine(const void* x0, int64_t p0, int32_t c0, const void* x1,

@@ -288,6 +288,26 @@ def test_fp32_group_norm_of_large_tensors(pkg, dev, shape, c1, groups, mean) -> 
     np.testing.assert_allclose(aff, want, rtol=2e-6, atol=2e-6 + 2.0 ** -20 * abs(mean))
 
 
+@pytest.mark.parametrize(("shape", "c1"), [((1, 8, 16, 33, 16), 0), ((2, 17, 19, 23, 48), 16), ((1, 4, 9, 13, 6), 0),
+                                           ((1, 11, 13, 40, 6), 3)])
+@pytest.mark.parametrize("mean", [1e20, -3e37, 1e38])
+def test_fp32_group_norm_of_huge_values(pkg, dev, shape, c1, mean) -> None:
+    """Values whose squares overflow, with deviations whose squares do not: statistics as small
+    tensors' (one launch) have them, finite and within 2^-20 of the values. (Scale: 1 / deviation.)"""
+    rng = np.random.default_rng(8)
+    dev_ = 1e16
+    x = (mean + rng.normal(size=shape) * dev_).astype(np.float32)
+    c, groups = shape[-1], 2
+    x0, x1 = dev32(x[..., :c - c1], dev), dev32(x[..., c - c1:], dev) if c1 else None
+    gamma = dev32(np.full(c, 1e-3), dev)
+    aff = host(pkg.ops.group_norm_affine(x0, gamma, dev32(np.zeros(c), dev), groups=groups, eps=1e-5, x1=x1))
+    g64 = x.astype(np.float64).reshape(shape[0], -1, groups, c // groups)
+    std, mu = (np.repeat(f(g64, axis=(1, 3)), c // groups, axis=1) for f in (np.std, np.mean))
+    if dev_ > 2 ** -20 * abs(mean):   # the deviations are more than the values' rounding
+        np.testing.assert_allclose(aff[..., 0], 1e-3 / std, rtol=1e-4)
+    np.testing.assert_allclose(-aff[..., 1] / aff[..., 0], mu, rtol=2.0 ** -20)
+
+
 @pytest.mark.parametrize("batch", [2, 5])
 def test_fp32_group_norm_of_an_item_does_not_depend_on_its_batch(pkg, dev, batch) -> None:
     """Each item's statistics in the two-launch form: the bits of that item alone."""
