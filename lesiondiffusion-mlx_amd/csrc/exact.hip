@@ -548,7 +548,7 @@ __global__ __launch_bounds__(256) void attention_split_kernel(SplitAttnParams p)
 // it), seen on the sum that is needed anyway, so that no maximum is taken and the accumulators
 // are rarely rescaled; the block's probabilities are then made again. Probabilities are split as
 // in the kernel above, hi = half(p), lo = half((p - hi) 2^11), by packed conversions (an unscaled lo
-// is subnormal for small probabilities: 2.3e-5 of a sum of many at 2^-18, 3e-6 scaled).
+// is subnormal for small probabilities: 2.3e-5 of a sum of many at 2^-18, under 4e-6 scaled).
 // Ph Vh has one accumulator, 2^11 (Pl Vh + Ph Vl) the other.
 // Per 32 x 32 block 12 (D = 32) MFMAs and about 110 VALU operations, 16 of them exp2; VALU-bound.
 // 23,104 tokens, two 32-wide heads: 1248 -> 481 us (284 TFLOP/s of FP32 products).

@@ -105,11 +105,13 @@ def test_config_sized_search_on_sampled_rows(pkg, dev, dtype) -> None:
 
 
 @pytest.mark.parametrize("dtype", list(DTYPES))
-@pytest.mark.parametrize(("positions", "entries"), [(81920, 64), (82001, 2049), (81919, 4130), (97, 6143), (33, 65)])
+@pytest.mark.parametrize(("positions", "entries"), [(81920, 64), (82001, 2049), (81919, 4130), (97, 6143), (33, 65),
+                                                    (24576, 64), (24577, 2049), (24576, 4130)])
 def test_search_edges_of_chunks_and_schedules(pkg, dev, dtype, positions, entries) -> None:
-    """Both schedules around their boundary (81,920 positions) and code counts around the
-    64-code chunks and 2,048-code stages; duplicates across chunks, values near zero and large,
-    an all-zero and a non-finite latent: sampled rows and the last ones equal the oracle."""
+    """Both schedules around their boundaries (fp16: whole scans from 81,920 positions; FP32: bounds
+    above 24,576) and code counts around the 64-code chunks and 2,048-code stages; duplicates
+    across chunks, values near zero and large, an all-zero and a non-finite latent: sampled rows
+    and the last ones equal the oracle."""
     tt, nt = DTYPES[dtype]
     rng = np.random.default_rng(positions + entries)
     cb = (rng.normal(size=(entries, 4)) * np.exp2(rng.integers(-12, 5, (entries, 1)))).astype(nt)
@@ -200,3 +202,33 @@ def test_search_beyond_the_normal_range(pkg, dev, kind, positions) -> None:
     if kind == "doubled dot overflows":
         assert want[0] == 100 and want[1] == 77
     np.testing.assert_array_equal(idx, want)
+
+
+@pytest.mark.parametrize("positions", [3000, 24700])
+@pytest.mark.parametrize("scale", [2.0 ** -20, 1.0, 1e5])
+def test_search_of_near_ties_between_chunks(pkg, dev, positions, scale) -> None:
+    """Pairs of codes in different 64-code chunks (every fourth pair with a third) at the same distance
+    to the latents but for a few ulps of the distance, at norms 200 times that distance, where
+    the bounds are widest beside it: every row equals the oracle's."""
+    rng = np.random.default_rng(positions)
+    cb = rng.normal(size=(192, 4))
+    cb *= 60 / np.linalg.norm(cb, axis=1, keepdims=True)
+    unit = lambda v: v / np.linalg.norm(v, axis=-1, keepdims=True)  # noqa: E731
+    n = 24
+    centre, u = 8 * unit(rng.normal(size=(n, 4))), unit(rng.normal(size=(n, 4)))
+    v = rng.normal(size=(n, 4))
+    v = unit(v - (v * u).sum(1, keepdims=True) * u)
+    cb[:n], cb[128:128 + n] = centre + 0.5 * u, centre - 0.5 * u
+    cb[64:64 + n:4] = (centre + 0.5 * v)[::4]
+    i = rng.integers(0, n, positions)
+    w = rng.normal(size=(positions, 4))
+    for axis in (u[i], v[i] - (v[i] * u[i]).sum(1, keepdims=True) * u[i]):   # w orthogonal to u and v
+        w -= (w * axis).sum(1, keepdims=True) * axis
+    ulp = 2.0 ** -17   # of the norms' sum, 128, in FP32
+    flat = centre[i] + 0.2 * unit(w) + u[i] * rng.integers(-4, 5, (positions, 1)) * ulp / 2
+    cb, flat = (cb * scale).astype(np.float32), (flat * scale).astype(np.float32)
+    idx, _, _ = _search(pkg, dev, flat, cb, torch.float32)
+    d = ovq.distances4(flat, cb, np.float32)
+    two = np.sort(d, axis=1)[:, :2].astype(np.float64)
+    assert np.median(two[:, 1] - two[:, 0]) <= 4 * ulp * scale ** 2
+    np.testing.assert_array_equal(idx, np.argmin(d, axis=1))
