@@ -12,7 +12,8 @@
 // The dots run on the matrix units: v_mfma_f32_32x32x2_f32 adds its two products in order, each
 // as one fp32 fused multiply-add (tests compare every index and value with the fma chain), so
 // two of them give the reference's chain for 32 codes x 32 positions (its first product plain
-// up to the sign of a zero, which no distance shows). Integer/index results are bit-exact.
+// up to the sign of a zero, which no distance shows). A few codes are scanned on the VALU.
+// Integer/index results are bit-exact.
 
 #include "common.h"
 
@@ -566,6 +567,66 @@ __global__ __launch_bounds__(VQ_THREADS, 4) void vq_nearest4_bounds_kernel(
   }
 }
 
+// Few codes: a lane per position scans them all with the reference's operations, from LDS reads that
+// all lanes share, eight codes at a time. The searches above cost a stage, a merge and a second pass
+// whatever the codes' number (9.6 us for one code, 44 at 409,600 positions); this one thirteen VALU
+// operations a pair and nothing else: VALU-bound from 200,000 positions on, one wave's chain (0.04
+// us a code) below 100,000.
+constexpr int VQ_SCAN_CODES = 256;
+static_assert(VQ_SCAN_CODES <= VQ_THREADS && VQ_SCAN_CODES % 8 == 0, "a code per thread, whole eights");
+template <typename T>
+__global__ __launch_bounds__(VQ_THREADS) void vq_scan4_kernel(
+    const T* __restrict__ z, const T* __restrict__ z_norm, const T* __restrict__ codebook,
+    const T* __restrict__ cb_norm, int64_t P, int E, int32_t* __restrict__ indices, T* __restrict__ quantized) {
+  __shared__ float4 cb[VQ_SCAN_CODES];
+  __shared__ T cbn[VQ_SCAN_CODES];
+  const int64_t pos = (int64_t)blockIdx.x * VQ_THREADS + threadIdx.x;
+  const int nr = (E + 7) / 8 * 8;   // whole eights: the last code again, which never wins twice
+  if ((int)threadIdx.x < nr) {
+    const int i = min((int)threadIdx.x, E - 1);
+    const T* e = codebook + (int64_t)i * 4;
+    cb[threadIdx.x] = make_float4((float)e[0], (float)e[1], (float)e[2], (float)e[3]);
+    cbn[threadIdx.x] = cb_norm[i];
+  }
+  __syncthreads();
+  if (pos >= P) return;
+  T zt[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) zt[c] = z[pos * 4 + c];
+  const T zn = z_norm ? z_norm[pos] : squared_norm4<T>(zt);
+  auto distance = [&](int code) {
+    const float4 e = cb[code];
+    float dot = (float)zt[0] * e.x;
+    dot = __builtin_fmaf((float)zt[1], e.y, dot);
+    dot = __builtin_fmaf((float)zt[2], e.z, dot);
+    dot = __builtin_fmaf((float)zt[3], e.w, dot);
+    if constexpr (sizeof(T) == 2) asm("" : "+v"(dot));   // as in code_distance
+    return vq_distance<T>(zn, cbn[code], dot);
+  };
+  T best = distance(0);
+  int found = 0;
+  for (int code = 0; code < nr; code += 8) {
+    T d[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) d[i] = distance(code + i);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const bool better = ((d[i] != d[i]) & (best == best)) | (d[i] < best);
+      best = better ? d[i] : best;
+      found = better ? code + i : found;
+    }
+  }
+  indices[pos] = found;
+  if (quantized) {
+#pragma unroll
+    for (int c = 0; c < 4; c++) quantized[pos * 4 + c] = (T)(zt[c] + (T)(codebook[found * 4 + c] - zt[c]));
+  }
+}
+
+// Few codes: the scan. us, scan / the search below: 64 codes 1,000 positions 4.7 / 9.6, 409,600 9.8 /
+// 45 (fp16 11 / 45); 128 codes 1,000 7.4 / 9.6 (fp16 8.1 / 9.7), 409,600 17 / 45; 256 codes 50,000
+// 13.3 / 13.5 (fp16 14.9 / 20), 100,000 14.3 / 18.2, 409,600 31 / 46 (fp16 34 / 56); 384 codes lose at
+// 50,000 (18 estimated / 14).
 // Up to 24,576 positions the quarters' workgroups run at once (three per CU), whole scans leave
 // waves idle. FP32 above that: bounds. us, quarters / bounds, 8,192 codes: 500 positions 34 / 45,
 // 24,000 46 / 76, 28,000 77 / 45, 51,200 111 / 75, 100,000 163 / 75 (whole exact scans); 24,000 x
@@ -576,6 +637,11 @@ template <typename T>
 static void launch_vq_nearest4(const T* z, const T* z_norm, const T* codebook, const T* cb_norm, int64_t P, int E,
                                int32_t* indices, T* quantized, hipStream_t st) {
   constexpr bool F32 = sizeof(T) == 4;
+  if (E <= 128 || (E <= VQ_SCAN_CODES && P > 32768)) {
+    hipLaunchKernelGGL(vq_scan4_kernel<T>, dim3((unsigned)((P + VQ_THREADS - 1) / VQ_THREADS)), dim3(VQ_THREADS), 0, st,
+                       z, z_norm, codebook, cb_norm, P, E, indices, quantized);
+    return;
+  }
   if (P <= (F32 ? 24576 : 81919)) {
     hipLaunchKernelGGL((vq_nearest4_kernel<T, 1, 4>), dim3((unsigned)((P + 31) / 32)), dim3(VQ_THREADS), 0, st, z,
                        z_norm, codebook, cb_norm, P, E, indices, quantized);

@@ -126,6 +126,47 @@ def test_search_edges_of_chunks_and_schedules(pkg, dev, dtype, positions, entrie
     np.testing.assert_array_equal(_bits(q[rows][:-4]), _bits(want_q[:-4]))
 
 
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize(("positions", "entries"), [(1, 1), (300, 2), (257, 63), (257, 64), (24577, 128), (24577, 129),
+                                                    (32768, 256), (32769, 256), (32769, 250), (81920, 249),
+                                                    (32769, 257)])
+def test_search_of_few_codes(pkg, dev, dtype, positions, entries) -> None:
+    """Codebooks on both sides of the scan's boundaries, with duplicates, a non-finite code in every
+    third case, zeros and infinite latents: sampled rows and the last ones equal the oracle."""
+    tt, nt = DTYPES[dtype]
+    rng = np.random.default_rng(positions + entries)
+    cb, flat = rng.normal(size=(entries, 4)).astype(nt), rng.normal(size=(positions, 4)).astype(nt)
+    cb[-1] = cb[entries // 2]
+    if entries > 2 and (positions + entries) % 3 == 0:
+        cb[entries - 2, 1] = np.inf
+    if positions > 4:
+        flat[-1], flat[-2], flat[-3, 0], flat[-4, 1] = cb[0], 0, np.inf, np.nan
+    idx, q, _ = _search(pkg, dev, flat, cb, tt)
+    rows = np.unique(np.concatenate([[0], np.maximum(positions - 1 - np.arange(300), 0), rng.integers(0, positions, 512)]))
+    with np.errstate(invalid="ignore", over="ignore"):
+        want_idx, want_q = ovq.quantize4(flat[rows], cb, nt)
+    np.testing.assert_array_equal(idx[rows], want_idx)
+    ok = ~np.isnan(want_q)
+    np.testing.assert_array_equal(np.isnan(q[rows]), ~ok)
+    np.testing.assert_array_equal(_bits(q[rows])[ok], _bits(want_q)[ok])
+
+
+@pytest.mark.parametrize(("positions", "entries"), [(40, 8192), (82000, 8192), (82000, 200)])
+def test_half_dots_are_rounded_to_fp32_first(pkg, dev, positions, entries) -> None:
+    """fp16 latents whose chosen code depends on the dot's rounding to fp32 before fp16 (one fused
+    rounding gives another index): every schedule takes the oracle's."""
+    rng = np.random.default_rng(417792)
+    cb, flat = (rng.normal(size=(n, 4)).astype(np.float32).astype(np.float16) for n in (8192, 409600))
+    flat = np.resize(flat[[15652, 277019, 392416]], (positions, 4))
+    if entries < 8192:
+        cb = np.concatenate([cb[[7303, 7232, 2805, 3631, 6794, 5333]], cb[:entries - 6]])
+    idx, _, _ = _search(pkg, dev, flat, cb, torch.float16)
+    want, _ = ovq.quantize4(flat[:3], cb, np.float16)
+    if entries == 8192:
+        np.testing.assert_array_equal(want, [7232, 3631, 5333])
+    np.testing.assert_array_equal(idx, np.resize(want, positions))
+
+
 def test_search_rejects_bad_arguments(pkg, dev) -> None:
     """Shape and dtype errors raise before anything is launched."""
     z = torch.zeros((3, 4), dtype=torch.float16, device=dev)
