@@ -1472,6 +1472,22 @@ static int launch_narrow(ExactConvParams p, int64_t bricks, hipStream_t st) {
 
 static bool al16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
+// Whether a conv with an odd number of 32-channel output blocks takes the 32- / 16-row kernel:
+// `nb` bricks of 128 voxels, `wide` workgroups of the 64-row kernel with them, `small` with its
+// bricks of 32. A narrow workgroup walks the input channels in one chain (the 64-row kernel
+// splits them over k-groups), so from 33 channels on it needs the other's workgroups to be many:
+// us, 64-row tile / narrow, 16x16x32 (64 bricks) 64->32 15.6 / 25.8, 256->32 36 / 89; 17x29x23 (120)
+// 128->32 39 / 47 but 96->16 36 / 28; one round of the 64-row tile 16x32x64 64->32 32 / 26, 128->32 56
+// / 68, 256->32 101 / 146, 16x16x64 256->96 108 / 158; more rounds 20x32x64 128->32 107 / 75, 256->32
+// 201 / 146, 256->160 413 / 447, 17x29x23 128->224 112 / 151.
+static bool narrow_pays(int C, int O, int64_t nb, int64_t wide, int64_t small) {
+  if (nb < 64) return false;
+  if (C <= 32) return true;
+  if (wide < 128) return O <= 16 && C <= 128 && small > 256;
+  if (wide <= 256) return C <= 64 || (C <= 128 && (O <= 16 || nb * ((O + 31) / 32) <= 240));
+  return C <= 128 ? O <= 160 || wide > 512 : O <= 96;
+}
+
 int conv3d_exact(const ldx_conv3d_args* a, void* stream) {
   int64_t rg[3], og[3];
   if (int rc = exact_geometry(a, rg, og)) return rc;
@@ -1523,8 +1539,8 @@ int conv3d_exact(const ldx_conv3d_args* a, void* stream) {
     return launch_exact<3, 2, 2, 4, 4, 2, 1>(p, nb, st);
   }
   // An odd number of 32-channel output blocks leaves the 64-row tile half empty (O <= 16:
-  // three quarters): those take the 32- / 16-row kernel from 64 bricks on (its loads need
-  // 16-byte rows, a concat on a 16-channel boundary and 31-bit offsets over a halo's planes).
+  // three quarters): those take the 32- / 16-row kernel where it pays (its loads need 16-byte
+  // rows, a concat on a 16-channel boundary and 31-bit offsets over a halo's planes).
   // us, 64-row tile / narrow, GroupNorm + SiLU and residual: 76x128x152 16->16 854 / 151 and
   // 32->16 873 / 273; 38x64x76 32->32 147 / 64; 19x32x38 64->32 32 / 26; 20x24x24 32->32
   // 25 / 16; 40x64x64 96->96 438 / 345. Whole pairs of blocks stay: 19x32x38 128->64 60 / 72,
@@ -1536,8 +1552,9 @@ int conv3d_exact(const ldx_conv3d_args* a, void* stream) {
       nb = bricks(4, 8, 8);
       if (nb >= 64) return launch_narrow<16, 4, 8, 1>(p, nb, st);
     }
+    const int64_t small = bricks(2, 4, 4) * oblocks;   // workgroups of the wide kernel's 32-voxel brick
     nb = bricks(4, 4, 8);
-    if (nb >= 64)
+    if (narrow_pays(C, O, nb, nb * oblocks, small))
       return O <= 16 ? launch_narrow<16, 4, 4, 2>(p, nb, st)
              : C <= 16 ? launch_narrow<32, 4, 4, 1>(p, nb, st) : launch_narrow<32, 4, 4, 2>(p, nb, st);
   }

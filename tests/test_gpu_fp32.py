@@ -148,9 +148,12 @@ def test_fp32_exact_conv_tilings_with_group_norm_prologue(pkg, dev, shape, out_c
     ((1, 8, 16, 17, 57), 8, 32, False, None),      # half a chunk, 32 rows
     ((1, 20, 5, 9, 17), 20, 32, True, None),       # the upsampled grid
     ((1, 64, 16, 16, 36), 32, 96, False, None),    # three row blocks
+    ((1, 96, 17, 18, 33), 48, 16, False, None),    # six chunks, 125 bricks
+    ((1, 96, 16, 15, 33), 96, 32, False, None),    # 80 bricks: the 64-row tile's four k-groups
+    ((1, 160, 16, 16, 60), 160, 32, False, "silu"),  # 128 bricks: the 64-row tile's two
 ])
 def test_fp32_narrow_output_conv(pkg, dev, shape, c0, out_c, up, act) -> None:
-    """The 16- and 32-row tiles (at least 64 bricks of 4 x 4 x 8) at the exact-mode bound,
+    """The 16- and 32-row tiles, and the 64-row ones where they are faster, at the exact-mode bound,
     through the GroupNorm affine + SiLU prologue and the whole epilogue."""
     x, w, _ = fp32_case(shape, out_c, sum(shape) + out_c)
     rng = np.random.default_rng(out_c + c0)
