@@ -1417,14 +1417,16 @@ static int plan_conv(const ldx_conv3d_args* a, ConvParams& p, Tile& t, size_t& l
   // us, 64 x 256 / 96 x 256 tiles, GroupNorm + SiLU + residual: 128x160x160 96->96 2241 / 1622
   // (1,005 TFLOP/s), 64x80x80 96->96 280 / 214 and 288->288 1991 / 1635, 50x61x70 96->96 328 / 123 (the
   // 64-row tile's brick of least waste has a long halo there), 36x60x62 115 / 97, 30x50x52 (below
-  // 512 workgroups) the same.
+  // 512 workgroups) the same. A gain of less than a twentieth in slots is lost to the three chains
+  // per wave: 88x100x12 256->96, 0.96 of the slots, 174 / 188.
   if (p.taps == 27 && p.stride == 1 && vec && p.O > 64 && (p.C1 == 0 || p.C0 % 32 == 0)) {
     const int64_t o96 = (p.O + 95) / 96, o64 = (p.O + 63) / 64;
     int bd, bh, bw, td, th, tw;
     const int64_t s96 = pick_brick96(p, td, th, tw);
     pick_brick(p, 256, 1, 3, bd, bh, bw);
     const int64_t s64 = ceil_div64(p.RD, bd) * ceil_div64(p.RH, bh) * ceil_div64(p.RW, bw) * 256;
-    if (o96 * 96 < o64 * 64 && s96 * o96 * 96 <= s64 * o64 * 64 && s96 / 256 * o96 * p.B >= 512) t = {1, 4, 3, 2, 32};
+    if (o96 * 96 < o64 * 64 && 20 * s96 * o96 * 96 <= 19 * s64 * o64 * 64 && s96 / 256 * o96 * p.B >= 512)
+      t = {1, 4, 3, 2, 32};
   }
   // LDX_CONV_TILE="WO,WV,FO,FV,CC" overrides the tile heuristic (tuning sweeps).
   bool forced = false;
