@@ -1216,28 +1216,36 @@ struct Tile {
   int BV() const { return WV * FV * 32; }
 };
 
-static void pick_brick(const ConvParams& p, int BV, int s, int ks, int& TD, int& TH, int& TW) {
+static void pick_brick(const ConvParams& p, int64_t per, int BV, int s, int ks, int& TD, int& TH, int& TW) {
   // Minimise launched voxel slots (partial-brick waste) plus a quarter of the halo voxels staged
   // (what a halo voxel's staging costs beside a slot's MFMAs), then the halo volume. By slots
   // alone ragged volumes got long bricks with halos of four voxels per output: us, before / now,
   // 61x77x83 32->32 73 / 48, 50x61x70 96->32 141 / 68, 53x71x34 256->256 stride 2 400 / 333, upsampling
   // 41x33x57 64->32 136 / 76; weights of 0.1 to 0.5 within 5 % of each other.
-  int64_t best_cost = INT64_MAX, best_halo = INT64_MAX;
+  struct Brick { int d, h, w; int64_t nb, halo; };
+  Brick best{}, least{};   // by that cost, by slots
   for (int td = 1; td <= BV; td *= 2)
     for (int th = 1; td * th <= BV; th *= 2) {
       const int tw = BV / (td * th);
-      if (td * th * tw != BV) continue;
       const int64_t nb = ceil_div64(p.RD, td) * ceil_div64(p.RH, th) * ceil_div64(p.RW, tw);
-      const int64_t slots = nb * BV;
       const int hd = ks == 1 ? td : (s == 2 ? 2 * td + 1 : td + 2);
       const int hh = ks == 1 ? th : (s == 2 ? 2 * th + 1 : th + 2);
       const int hw = ks == 1 ? tw : (s == 2 ? 2 * tw + 1 : tw + 2);
-      const int64_t halo = (int64_t)hd * hh * hw;
-      const int64_t cost = 4 * slots + nb * halo;
-      if (cost < best_cost || (cost == best_cost && halo < best_halo)) {
-        best_cost = cost; best_halo = halo; TD = td; TH = th; TW = tw;
-      }
+      const Brick b{td, th, tw, nb, (int64_t)hd * hh * hw};
+      auto cost = [&](const Brick& k) { return k.nb * (4 * BV + k.halo); };
+      if (!best.d || cost(b) < cost(best) || (cost(b) == cost(best) && b.halo < best.halo)) best = b;
+      if (!least.d || b.nb < least.nb || (b.nb == least.nb && b.halo < least.halo)) least = b;
     }
+  // With up to four workgroups per CU (`per` of them a brick) one more counts as a whole round of
+  // slots: the brick of fewest slots stays where the other would add one. us, that brick / the other:
+  // 39x34x93 64->32 (510, 540 workgroups) 29 / 39, 44x45x15 96->32 (253, 264) 13.5 / 16.7, 22x31x22
+  // 96->128 (484, 528) 23 / 26. (Not at stride 2, where the halo is most of the work: 75x52x29 256->256,
+  // 988 and 1,040 workgroups, 248 / 156.)
+  auto rounds = [&](const Brick& k) { return ceil_div64(k.nb * per, 256); };
+  auto whole = [&](const Brick& k) { return rounds(k) * 256 * 4 * BV + per * k.nb * k.halo; };
+  if (s == 1 && !p.upsample && rounds(least) <= 4 && rounds(least) < rounds(best) && whole(least) < whole(best))
+    best = least;
+  TD = best.d; TH = best.h; TW = best.w;
 }
 
 // Bricks of the 96-channel tile (256 voxels), whose halo beside the weight ring leaves two
@@ -1423,7 +1431,7 @@ static int plan_conv(const ldx_conv3d_args* a, ConvParams& p, Tile& t, size_t& l
     const int64_t o96 = (p.O + 95) / 96, o64 = (p.O + 63) / 64;
     int bd, bh, bw, td, th, tw;
     const int64_t s96 = pick_brick96(p, td, th, tw);
-    pick_brick(p, 256, 1, 3, bd, bh, bw);
+    pick_brick(p, o64 * p.B, 256, 1, 3, bd, bh, bw);
     const int64_t s64 = ceil_div64(p.RD, bd) * ceil_div64(p.RH, bh) * ceil_div64(p.RW, bw) * 256;
     if (o96 * 96 < o64 * 64 && 20 * s96 * o96 * 96 <= 19 * s64 * o64 * 64 && s96 / 256 * o96 * p.B >= 512)
       t = {1, 4, 3, 2, 32};
@@ -1449,7 +1457,7 @@ static int plan_conv(const ldx_conv3d_args* a, ConvParams& p, Tile& t, size_t& l
   int TD = 1, TH = 1, TW = 1;
   for (;;) {
     if (t.FO == 3) pick_brick96(p, TD, TH, TW);
-    else pick_brick(p, t.BV(), s, ks, TD, TH, TW);
+    else pick_brick(p, (p.O + t.BO() - 1) / t.BO() * (int64_t)p.B * (p.upsample ? 8 : 1), t.BV(), s, ks, TD, TH, TW);
     p.TD = TD; p.TH = TH; p.TW = TW;
     p.HD = ks == 1 ? TD : (s == 2 ? 2 * TD + 1 : TD + 2);
     p.HH = ks == 1 ? TH : (s == 2 ? 2 * TH + 1 : TH + 2);
